@@ -29,6 +29,10 @@
 // the r, s and lambda parts, D_t the derivative along k),
 // q . A_L q = q . P + (D_t q) . Gqt = sum of q P + qt Gqt over the nodes, so
 // no q has to outlive phase K. The E-vector is the same, bit for bit.
+//
+// LAM = false (lambda = 0) does not read wJ: the mass term is +-0 with any
+// finite wJ, and the kernel streams 60 instead of 68 bytes per node (a NaN or
+// infinite wJ is not seen either, as in the other degrees' kernel).
 #include "reduce.hpp"
 
 namespace libp_amd {
@@ -39,7 +43,7 @@ __device__ inline d4 mfma16(double a, double b, d4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-template <bool PAP>
+template <bool PAP, bool LAM>
 __global__ void __launch_bounds__(256, 1) ax_hex_mfma_n15_kernel(const int* __restrict__ elementList,
                                                                  const int* __restrict__ G2L,
                                                                  const double* __restrict__ wJ,
@@ -98,7 +102,7 @@ __global__ void __launch_bounds__(256, 1) ax_hex_mfma_n15_kernel(const int* __re
       const int n = k * NqNq + (4 * r + lg) * Nq + li;
 #pragma unroll
       for (int g = 0; g < 6; ++g) Gn[g][r] = __builtin_nontemporal_load(gbase + g * Np + n);
-      Wn[r] = __builtin_nontemporal_load(wbase + n);
+      if (LAM) Wn[r] = __builtin_nontemporal_load(wbase + n);
     }
   };
   loadG(4 * w);
@@ -125,7 +129,7 @@ __global__ void __launch_bounds__(256, 1) ax_hex_mfma_n15_kernel(const int* __re
     for (int r = 0; r < 4; ++r) {
 #pragma unroll
       for (int g = 0; g < 6; ++g) G[g][r] = Gn[g][r];
-      W[r] = Wn[r];
+      if (LAM) W[r] = Wn[r];
     }
     if (kk < 3) loadG(k + 1);
     d4 qr = {0, 0, 0, 0}, qs = {0, 0, 0, 0};
@@ -146,7 +150,7 @@ __global__ void __launch_bounds__(256, 1) ax_hex_mfma_n15_kernel(const int* __re
       Gqs[r] = G[1][r] * qr[r] + G[3][r] * qs[r] + G[4][r] * qt;
       const double Gqt = G[2][r] * qr[r] + G[4][r] * qs[r] + G[5][r] * qt;
       s_t[n] = Gqt;  // in place
-      lam[r] = W[r] * lambda * qn;
+      if (LAM) lam[r] = W[r] * lambda * qn;
       s_x[w][(4 * r + lg) * Nq + li] = Gqr[r];
       if (PAP) {
         qk[r] = qn;
@@ -166,7 +170,7 @@ __global__ void __launch_bounds__(256, 1) ax_hex_mfma_n15_kernel(const int* __re
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const double P = acc[r] + lam[r];
+      const double P = LAM ? acc[r] + lam[r] : acc[r];
       s_q[k * NqNq + (4 * r + lg) * Nq + li] = P;
       if (PAP) papAcc += qk[r] * P;
     }
@@ -200,8 +204,9 @@ __global__ void __launch_bounds__(256, 1) ax_hex_mfma_n15_kernel(const int* __re
 int launch_ax_mfma_n15_pap(int Nelements, const int* elementList, const int* G2L, const double* wJ,
                            const double* ggeo, const double* D, double lambda, const double* p, double* AqL,
                            double* part, const double* scal, hipStream_t st) {
-  hipLaunchKernelGGL(ax_hex_mfma_n15_kernel<true>, dim3(Nelements), dim3(256), 0, st, elementList, G2L, wJ, ggeo, D,
-                     lambda, p, AqL, part, scal);
+  const auto kernel = lambda != 0.0 ? ax_hex_mfma_n15_kernel<true, true> : ax_hex_mfma_n15_kernel<true, false>;
+  hipLaunchKernelGGL(kernel, dim3(Nelements), dim3(256), 0, st, elementList, G2L, wJ, ggeo, D, lambda, p, AqL, part,
+                     scal);
   return launch_status("pcg_ax_hex_pap (N=15)");
 }
 
@@ -214,7 +219,8 @@ extern "C" int libp_ax_hex_partial_mfma_n15(int Nelements, const int* elementLis
                                             const double* q, double* AqL, void* stream) {
   if (Nelements <= 0) return LIBP_OK;
   if (!GlobalToLocal || !wJ || !ggeo || !D || !q || !AqL) return arg_error("ax_hex_mfma_n15", "null pointer");
-  hipLaunchKernelGGL(ax_hex_mfma_n15_kernel<false>, dim3(Nelements), dim3(256), 0, as_stream(stream), elementList,
-                     GlobalToLocal, wJ, ggeo, D, lambda, q, AqL, nullptr, nullptr);
+  const auto kernel = lambda != 0.0 ? ax_hex_mfma_n15_kernel<false, true> : ax_hex_mfma_n15_kernel<false, false>;
+  hipLaunchKernelGGL(kernel, dim3(Nelements), dim3(256), 0, as_stream(stream), elementList, GlobalToLocal, wJ, ggeo, D,
+                     lambda, q, AqL, nullptr, nullptr);
   return launch_status("ax_hex_mfma_n15");
 }
