@@ -10,11 +10,21 @@
 // lane, so the product does not depend on how the hardware orders K inside it.
 //
 // Tiles: 128x128 per workgroup of four wavefronts (2x2, 64x64 each = 2x2
-// MFMA blocks), BK = 32, two LDS buffers with register prefetch of the next
-// K tile. Operands reach LDS as [row][k] (row stride 40 elements) whatever
+// MFMA blocks), BK = 64, two LDS buffers with register prefetch of the next
+// K tile, two workgroups per CU (the layers have 512 to 1024 tiles).
+// What bounds it: the LDS reads of a K tile take as long as its MFMAs, and with
+// two workgroups per CU little covers a tile's first loads and its epilogue.
+// 32,768 rows, microseconds before -> now: forward 896->256 37 -> 26 (0.58
+// PFLOP/s), 256->256 22 -> 14, 256->512 26 -> 25; data gradient 512->256 42 -> 22,
+// 256->256 33 -> 16; weight gradient 256x896 92 -> 34, 256x256 75 -> 15,
+// 512x256 78 -> 21; the column and split sums of the three 275 -> 40. Operands reach LDS as [row][k] (row stride 40 elements) whatever
 // their layout in HBM: a K-contiguous operand is copied with 16-byte loads and
-// stores, a row-contiguous one (the transposed operands of the weight
-// gradients) with 16-byte loads and 2-byte LDS stores.
+// stores; of a row-contiguous one (the transposed operands of the backward
+// products) each thread loads a 4 x 4 patch, four 8-byte loads, transposes it
+// with byte permutes and stores four 8-byte pieces. (With 16-byte loads and
+// sixteen 2-byte LDS stores per thread the LDS writes bound the kernel: dW of
+// 32,768 x 896 x 256 took 92 us, and 32,768 x 256 x 256 took 75.)
+#include <algorithm>
 #include <cmath>
 
 #include "reduce.hpp"
@@ -25,6 +35,8 @@ typedef unsigned short u16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // float -> bf16, round to nearest even; NaN stays NaN
 __device__ inline u16 f2bf(float f) {
@@ -35,7 +47,7 @@ __device__ inline u16 f2bf(float f) {
 }
 __device__ inline float bf2f(u16 h) { return __builtin_bit_cast(float, (unsigned)h << 16); }
 
-constexpr int GBM = 128, GBN = 128, GBK = 32, GLD = GBK + 8;
+constexpr int GBM = 128, GBN = 128, GBK = 64, GLD = GBK + 8;
 constexpr int GTHREADS = 256;
 
 enum { EPI_F32_BIAS = 0, EPI_BF16_BIAS_RELU = 1, EPI_BF16_MASK = 2, EPI_F32_PARTIAL = 3 };
@@ -55,38 +67,52 @@ struct GemmArgs {
   const float* rowScale = nullptr;  // EPI_F32_BIAS: C[m][n] = rowScale[m] * (A B + bias)[m][n] when set
 };
 
-// One operand tile (rows x GBK) in registers: two 16-byte chunks per thread.
+// One operand tile (rows x GBK) in registers: GCH 16-byte chunks per thread.
+constexpr int GCH = GBM * GBK * 2 / 16 / GTHREADS;
 struct TileRegs {
-  u32x4 v[2];
+  u32x4 v[GCH];
 };
 
+// A tile inside the matrix (and aligned: vec) takes loads that no branch guards,
+// so that they are all in flight together; the others take them entry by entry.
 template <bool T>
 __device__ inline void load_tile(TileRegs& R, const u16* __restrict__ X, long ld, int row0, int nrows, int k0, int kEnd,
                                  bool vec) {
   const int t = threadIdx.x;
+  const bool whole = vec && row0 + GBM <= nrows && k0 + GBK <= kEnd;  // the same for every thread
+  if (T) {  // patch i: rows k0 + 32 i + 4 (t & 7) + r, r = 0..3; columns row0 + 4 (t >> 3) ..
+    const int gk0 = k0 + 4 * (t & 7), gr = row0 + 4 * (t >> 3);
+    if (whole) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int c = t + GTHREADS * i;
-    u16 tmp[8];
-    if (!T) {
-      const int row = c >> 2, kc = (c & 3) * 8;
-      const int gr = row0 + row, gk = k0 + kc;
-      if (vec && gr < nrows && gk + 8 <= kEnd) {
-        R.v[i] = *reinterpret_cast<const u32x4*>(X + (long)gr * ld + gk);
-        continue;
+      for (int ir = 0; ir < 2 * GCH; ++ir) {
+        const u32x2 w = *reinterpret_cast<const u32x2*>(X + (long)(gk0 + 32 * (ir >> 2) + (ir & 3)) * ld + gr);
+        R.v[ir >> 1][2 * (ir & 1)] = w.x;
+        R.v[ir >> 1][2 * (ir & 1) + 1] = w.y;
       }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) tmp[e] = (gr < nrows && gk + e < kEnd) ? X[(long)gr * ld + gk + e] : (u16)0;
-    } else {
-      const int kr = c >> 4, rc = (c & 15) * 8;
-      const int gk = k0 + kr, gr = row0 + rc;
-      if (vec && gk < kEnd && gr + 8 <= nrows) {
-        R.v[i] = *reinterpret_cast<const u32x4*>(X + (long)gk * ld + gr);
-        continue;
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) tmp[e] = (gk < kEnd && gr + e < nrows) ? X[(long)gk * ld + gr + e] : (u16)0;
+      return;
     }
+#pragma unroll
+    for (int ir = 0; ir < 2 * GCH; ++ir) {
+      const int gk = gk0 + 32 * (ir >> 2) + (ir & 3);
+      u16 e[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) e[j] = (gk < kEnd && gr + j < nrows) ? X[(long)gk * ld + gr + j] : (u16)0;
+      R.v[ir >> 1][2 * (ir & 1)] = (unsigned)e[0] | ((unsigned)e[1] << 16);
+      R.v[ir >> 1][2 * (ir & 1) + 1] = (unsigned)e[2] | ((unsigned)e[3] << 16);
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < GCH; ++i) {
+    const int c = t + GTHREADS * i;
+    const int gr = row0 + c / (GBK / 8), gk = k0 + (c % (GBK / 8)) * 8;
+    if (whole) {
+      R.v[i] = *reinterpret_cast<const u32x4*>(X + (long)gr * ld + gk);
+      continue;
+    }
+    u16 tmp[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) tmp[e] = (gr < nrows && gk + e < kEnd) ? X[(long)gr * ld + gk + e] : (u16)0;
     R.v[i] = u32x4{(unsigned)tmp[0] | ((unsigned)tmp[1] << 16), (unsigned)tmp[2] | ((unsigned)tmp[3] << 16),
                    (unsigned)tmp[4] | ((unsigned)tmp[5] << 16), (unsigned)tmp[6] | ((unsigned)tmp[7] << 16)};
   }
@@ -95,43 +121,60 @@ __device__ inline void load_tile(TileRegs& R, const u16* __restrict__ X, long ld
 template <bool T>
 __device__ inline void store_tile(const TileRegs& R, u16* __restrict__ s) {
   const int t = threadIdx.x;
+  if (T) {  // column j of the patch: k entries of four rows, low and high halves picked by byte
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int c = t + GTHREADS * i;
-    if (!T) {
-      const int row = c >> 2, kc = (c & 3) * 8;
-      *reinterpret_cast<u32x4*>(s + row * GLD + kc) = R.v[i];
-    } else {
-      const int kr = c >> 4, rc = (c & 15) * 8;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const unsigned w = R.v[i][e >> 1];
-        s[(rc + e) * GLD + kr] = (u16)((e & 1) ? (w >> 16) : (w & 0xffffu));
-      }
+    for (int ij = 0; ij < 2 * GCH; ++ij) {
+      const int i = ij >> 2, j = ij & 3, d = j >> 1;
+      u16* o = s + 4 * (t >> 3) * GLD + 32 * i + 4 * (t & 7);
+      const unsigned pick = (j & 1) ? 0x07060302u : 0x05040100u;
+      *reinterpret_cast<u32x2*>(o + j * GLD) = u32x2{
+          __builtin_amdgcn_perm(R.v[2 * i][2 + d], R.v[2 * i][d], pick),
+          __builtin_amdgcn_perm(R.v[2 * i + 1][2 + d], R.v[2 * i + 1][d], pick)};
     }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < GCH; ++i) {
+    const int c = t + GTHREADS * i;
+    const int row = c / (GBK / 8), kc = (c % (GBK / 8)) * 8;
+    *reinterpret_cast<u32x4*>(s + row * GLD + kc) = R.v[i];
   }
 }
 
-template <bool TA, bool TB, int EPI>
-__global__ void __launch_bounds__(GTHREADS, 4) gemm_bf16_kernel(const GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) u16 sA[2][GBM * GLD];
-  __shared__ __attribute__((aligned(16))) u16 sB[2][GBN * GLD];
-  const int t = threadIdx.x, w = t >> 6, l = t & 63;
-  const int wm = w >> 1, wn = w & 1;
-  // Workgroups are dispatched round-robin over the eight XCDs, each with its
-  // own L2. When the M tiles come in multiples of eight, the tiles are renamed
-  // so that the gridDim.x N tiles of one M tile run on one XCD, one after
-  // another: the A rows (the large operand) then reach that L2 once instead of
-  // once per N tile. The tiles and their arithmetic are unchanged.
-  int mt = blockIdx.y, nt = blockIdx.x;
-  if ((gridDim.y & 7) == 0) {
+// Workgroups are dispatched round-robin over the eight XCDs, each with its
+// own L2. When the M tiles come in multiples of eight, the tiles are renamed
+// so that the gridDim.x N tiles of one M tile run on one XCD, one after
+// another: the A rows (the large operand) then reach that L2 once instead of
+// once per N tile. In the same way the tiles of one K split run on one XCD
+// when the splits come in multiples of eight (weight gradients: both operands'
+// rows of the split are read by every tile). The tiles and their arithmetic
+// are unchanged.
+__device__ inline void gemm_tile(int& mt, int& nt, int& split) {
+  mt = blockIdx.y, nt = blockIdx.x, split = blockIdx.z;
+  if ((gridDim.z & 7) == 0) {
+    const int tiles = gridDim.x * gridDim.y;
+    const int b = blockIdx.x + gridDim.x * blockIdx.y + tiles * blockIdx.z, k = b >> 3, tile = k % tiles;
+    split = (k / tiles) * 8 + (b & 7);
+    nt = tile % gridDim.x;
+    mt = tile / gridDim.x;
+  } else if ((gridDim.y & 7) == 0) {
     const int b = blockIdx.x + gridDim.x * blockIdx.y;  // dispatch order within a K split
     const int k = b >> 3;
     nt = k % gridDim.x;
     mt = (k / gridDim.x) * 8 + (b & 7);
   }
+}
+
+template <bool TA, bool TB, int EPI>
+__global__ void __launch_bounds__(GTHREADS, 2) gemm_bf16_kernel(const GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) u16 sA[2][GBM * GLD];
+  __shared__ __attribute__((aligned(16))) u16 sB[2][GBN * GLD];
+  const int t = threadIdx.x, w = t >> 6, l = t & 63;
+  const int wm = w >> 1, wn = w & 1;
+  int mt, nt, split;
+  gemm_tile(mt, nt, split);
   const int m0 = mt * GBM, n0 = nt * GBN;
-  const int kBeg = blockIdx.z * g.kChunk;
+  const int kBeg = split * g.kChunk;
   const int kEnd = min(g.K, kBeg + g.kChunk);
   const bool vecA = (g.lda % 8) == 0 && ((uintptr_t)g.A & 15) == 0;
   const bool vecB = (g.ldb % 8) == 0 && ((uintptr_t)g.B & 15) == 0;
@@ -206,40 +249,330 @@ __global__ void __launch_bounds__(GTHREADS, 4) gemm_bf16_kernel(const GemmArgs g
           const bool keep = !g.mask || bf2f(g.mask[(long)row * g.ldm + col]) > 0.f;
           reinterpret_cast<u16*>(g.C)[(long)row * g.ldc + col] = f2bf(keep ? v : 0.f);
         } else {
-          reinterpret_cast<float*>(g.C)[(long)blockIdx.z * g.M * g.ldc + (long)row * g.ldc + col] = v;
+          reinterpret_cast<float*>(g.C)[(long)split * g.M * g.ldc + (long)row * g.ldc + col] = v;
         }
       }
     }
+}
+
+// The same product where every access can be a whole vector (gemm_vectors below
+// says when): no load or store sits under a branch, so the loads of the next K
+// tile are all in flight during a tile's MFMAs. (Guarded per chunk, as in
+// gemm_bf16_kernel, each load was its own branch and each of the 64 two-byte
+// result stores waited for the one before it.) Rows past the end of A or B
+// repeat the last one (their results are not stored); K entries past the end of
+// a transposed operand are zeroed on the way to LDS. The result tile goes
+// through LDS, so bias, mask and C are read and written 16 bytes at a time.
+//
+// In LDS the 16-byte chunk c of row n of a transposed operand sits at chunk
+// c ^ (n / 16 % 4): the operand is read row by row, 32 lanes along 256 contiguous bytes (with eight
+// rows per load, lanes across rows, every lane was a request of its own: dW of
+// 32,768 x 896 x 256 took 67 us), and its patches, 4 rows of the tile apart, then meet
+// on two lanes per bank instead of eight; the MFMA reads stay conflict-free.
+template <bool T>
+__device__ inline int gemm_chunk(const int row, const int c) {
+  return row * GLD + ((T ? c ^ (row >> 4 & 3) : c) << 3);
+}
+
+template <bool T>
+struct VecTile {
+  u32x4 v[GCH];
+  __device__ inline void load(const u16* __restrict__ X, const long ld, const int row0, const int nrows, const int k0,
+                              const int kEnd) {
+    const int t = threadIdx.x;
+    if (T) {  // patch i: rows k0 + 32 i + 4 (t / 32) + r, r = 0..3, columns row0 + 4 (t % 32) ..
+      const u16* x = X + min(row0 + 4 * (t & 31), nrows - 4);
+#pragma unroll
+      for (int ir = 0; ir < 2 * GCH; ++ir) {
+        const int gk = min(k0 + 32 * (ir >> 2) + 4 * (t >> 5) + (ir & 3), kEnd - 1);
+        const u32x2 w = *reinterpret_cast<const u32x2*>(x + (long)gk * ld);
+        v[ir >> 1][2 * (ir & 1)] = w.x;
+        v[ir >> 1][2 * (ir & 1) + 1] = w.y;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < GCH; ++i) {
+        const int c = t + GTHREADS * i;
+        const int gr = min(row0 + c / (GBK / 8), nrows - 1), gk = min(k0 + (c % (GBK / 8)) * 8, kEnd - 8);
+        v[i] = *reinterpret_cast<const u32x4*>(X + (long)gr * ld + gk);
+      }
+    }
+  }
+  __device__ inline void store(u16* __restrict__ s, const int k0, const int kEnd) {
+    const int t = threadIdx.x;
+    if (k0 + GBK > kEnd) {  // the last K tile of a split: entries past the end are zero
+#pragma unroll
+      for (int i = 0; i < GCH; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int gk = T ? k0 + 32 * (i >> 1) + 4 * (t >> 5) + 2 * (i & 1) + h
+                           : k0 + ((t + GTHREADS * i) % (GBK / 8)) * 8;
+          if (gk >= kEnd) v[i][2 * h] = v[i][2 * h + 1] = 0u;
+        }
+    }
+    if (T) {  // column j of the patch: k entries of four rows, low and high halves picked by byte
+#pragma unroll
+      for (int ij = 0; ij < 2 * GCH; ++ij) {
+        const int i = ij >> 2, j = ij & 3, d = j >> 1;
+        const unsigned pick = (j & 1) ? 0x07060302u : 0x05040100u;
+        u16* o = s + gemm_chunk<T>(4 * (t & 31) + j, 4 * i + (t >> 6)) + 4 * (t >> 5 & 1);
+        *reinterpret_cast<u32x2*>(o) = u32x2{__builtin_amdgcn_perm(v[2 * i][2 + d], v[2 * i][d], pick),
+                                             __builtin_amdgcn_perm(v[2 * i + 1][2 + d], v[2 * i + 1][d], pick)};
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < GCH; ++i) {
+        const int c = t + GTHREADS * i;
+        *reinterpret_cast<u32x4*>(s + gemm_chunk<T>(c / (GBK / 8), c % (GBK / 8))) = v[i];
+      }
+    }
+  }
+};
+
+constexpr int GCLD = GBN + 4;  // row stride of the result tile in LDS (FP32)
+
+template <bool TA, bool TB, int EPI>
+__global__ void __launch_bounds__(GTHREADS, 2) gemm_bf16_vec_kernel(const GemmArgs g) {
+  constexpr int ABYTES = 2 * 2 * GBM * GLD * 2, CBYTES = GBM * GCLD * 4;
+  __shared__ __attribute__((aligned(16))) char smem[ABYTES > CBYTES ? ABYTES : CBYTES];
+  u16* const sA = reinterpret_cast<u16*>(smem);
+  u16* const sB = sA + 2 * GBM * GLD;
+  const int t = threadIdx.x, w = t >> 6, l = t & 63;
+  const int wm = w >> 1, wn = w & 1;
+  int mt, nt, split;
+  gemm_tile(mt, nt, split);
+  const int m0 = mt * GBM, n0 = nt * GBN;
+  const int kBeg = split * g.kChunk;
+  const int kEnd = min(g.K, kBeg + g.kChunk);
+  const int nT = (kEnd > kBeg) ? (kEnd - kBeg + GBK - 1) / GBK : 0;
+
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  const int lr = l & 31, lc = l >> 5;
+  const auto product = [&](const int buf) {
+    const u16* a_s = sA + buf * GBM * GLD;
+    const u16* b_s = sB + buf * GBN * GLD;
+#pragma unroll
+    for (int ks = 0; ks < GBK; ks += 16) {
+      bf16x8 a[2], b[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        a[i] = *reinterpret_cast<const bf16x8*>(a_s + gemm_chunk<TA>(wm * 64 + i * 32 + lr, ks / 8 + lc));
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        b[j] = *reinterpret_cast<const bf16x8*>(b_s + gemm_chunk<TB>(wn * 64 + j * 32 + lr, ks / 8 + lc));
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+  };
+  if (nT > 0) {
+    VecTile<TA> ra;
+    VecTile<TB> rb;
+    ra.load(g.A, g.lda, m0, g.M, kBeg, kEnd);
+    rb.load(g.B, g.ldb, n0, g.N, kBeg, kEnd);
+    ra.store(sA, kBeg, kEnd);
+    rb.store(sB, kBeg, kEnd);
+    __syncthreads();
+    for (int it = 0; it + 1 < nT; ++it) {
+      const int k0 = kBeg + (it + 1) * GBK;
+      ra.load(g.A, g.lda, m0, g.M, k0, kEnd);
+      rb.load(g.B, g.ldb, n0, g.N, k0, kEnd);
+      // all of the loads go out before the MFMAs: left to itself the scheduler spreads them
+      // between, the last ones right before the stores that wait for them
+      __builtin_amdgcn_sched_barrier(0);
+      product(it & 1);
+      ra.store(sA + ((it & 1) ^ 1) * GBM * GLD, k0, kEnd);
+      rb.store(sB + ((it & 1) ^ 1) * GBN * GLD, k0, kEnd);
+      __syncthreads();
+    }
+    product((nT - 1) & 1);
+  }
+  __syncthreads();  // the tiles have been read: the result tile takes their place
+
+  float* const sC = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        sC[(wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3)) * GCLD + wn * 64 + j * 32 + lr] = acc[i][j][r];
+  __syncthreads();
+  constexpr bool BF = EPI == EPI_BF16_BIAS_RELU || EPI == EPI_BF16_MASK;
+  constexpr int W = BF ? 8 : 4, RC = GBN / W, STEP = GTHREADS / RC, NS = GBM / STEP;  // W columns per access
+  const int cc = (t % RC) * W, r0 = t / RC;
+  const int col = n0 + cc;
+  if (col >= g.N) return;
+  float bias[W];
+#pragma unroll
+  for (int e = 0; e < W; ++e)
+    bias[e] = (g.bias && (EPI == EPI_F32_BIAS || EPI == EPI_BF16_BIAS_RELU)) ? g.bias[col + e] : 0.f;
+  u32x4 mask[EPI == EPI_BF16_MASK ? NS : 1];
+  float scale[EPI == EPI_F32_BIAS ? NS : 1];
+  if (EPI == EPI_BF16_MASK && g.mask) {
+#pragma unroll
+    for (int k = 0; k < NS; ++k)
+      mask[k] = *reinterpret_cast<const u32x4*>(g.mask + (long)min(m0 + r0 + STEP * k, g.M - 1) * g.ldm + col);
+  }
+  if (EPI == EPI_F32_BIAS && g.rowScale) {
+#pragma unroll
+    for (int k = 0; k < NS; ++k) scale[k] = g.rowScale[min(m0 + r0 + STEP * k, g.M - 1)];
+  }
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+    const int lrow = r0 + STEP * k, row = m0 + lrow;
+    float v[W];
+#pragma unroll
+    for (int e = 0; e < W; e += 4) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(sC + lrow * GCLD + cc + e);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[e + j] = x[j];
+    }
+    if (row < g.M) {
+      if (BF) {
+        unsigned o[W];
+#pragma unroll
+        for (int e = 0; e < W; ++e) {
+          if (EPI == EPI_BF16_BIAS_RELU) {
+            o[e] = f2bf(fmaxf(v[e] + bias[e], 0.f));
+          } else {
+            const unsigned m = mask[k][e >> 1];
+            const bool keep = !g.mask || bf2f((u16)((e & 1) ? (m >> 16) : (m & 0xffffu))) > 0.f;
+            o[e] = f2bf(keep ? v[e] : 0.f);
+          }
+        }
+        *reinterpret_cast<u32x4*>(reinterpret_cast<u16*>(g.C) + (long)row * g.ldc + col) =
+            u32x4{o[0] | (o[1] << 16), o[2] | (o[3] << 16), o[4] | (o[5] << 16), o[6] | (o[7] << 16)};
+      } else {
+        f32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          o[e] = v[e];
+          if (EPI == EPI_F32_BIAS) {
+            o[e] = v[e] + bias[e];
+            if (g.rowScale) o[e] = scale[k] * o[e];
+          }
+        }
+        const long base = EPI == EPI_F32_PARTIAL ? (long)split * g.M * g.ldc : 0;
+        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(g.C) + base + (long)row * g.ldc + col) = o;
+      }
+    }
+  }
+}
+
+// Whether gemm_bf16_vec_kernel serves the product: pointers and leading dimensions
+// whole vectors, the vectors of the contiguous dimension whole inside the matrix.
+template <bool TA, bool TB, int EPI>
+static bool gemm_vectors(const GemmArgs& g) {
+  const auto on16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+  constexpr bool BF = EPI == EPI_BF16_BIAS_RELU || EPI == EPI_BF16_MASK;
+  const int W = BF ? 8 : 4;
+  const bool a = on16(g.A) && g.lda % 8 == 0 && (TA ? g.M % 4 == 0 : g.K % 8 == 0);
+  const bool b = on16(g.B) && g.ldb % 8 == 0 && (TB ? g.N % 4 == 0 : g.K % 8 == 0);
+  const bool c = on16(g.C) && g.ldc % W == 0 && g.N % W == 0 && (EPI != EPI_F32_PARTIAL || (g.M * g.ldc) % 4 == 0);
+  return a && b && c && (!g.mask || (on16(g.mask) && g.ldm % 8 == 0));
 }
 
 template <bool TA, bool TB, int EPI>
 static int gemm(const GemmArgs& g, int splits, void* stream, const char* where) {
   if (g.M <= 0 || g.N <= 0) return LIBP_OK;
   dim3 grid((g.N + GBN - 1) / GBN, (g.M + GBM - 1) / GBM, splits);
-  hipLaunchKernelGGL((gemm_bf16_kernel<TA, TB, EPI>), grid, dim3(GTHREADS), 0, as_stream(stream), g);
+  if (gemm_vectors<TA, TB, EPI>(g))
+    hipLaunchKernelGGL((gemm_bf16_vec_kernel<TA, TB, EPI>), grid, dim3(GTHREADS), 0, as_stream(stream), g);
+  else
+    hipLaunchKernelGGL((gemm_bf16_kernel<TA, TB, EPI>), grid, dim3(GTHREADS), 0, as_stream(stream), g);
   return launch_status(where);
 }
 
-// out[i] (+)= sum_s P[s*n + i], s in order (deterministic)
-__global__ void __launch_bounds__(256) sum_splits_kernel(const long n, const int S, const float* __restrict__ P,
-                                                         float* __restrict__ out) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    float a = 0.f;
-    for (int s = 0; s < S; ++s) a += P[(long)s * n + i];
-    out[i] = a;
+// Column sums of a BF16 [M][ld] matrix, two stages: block (x, y) sums 64 columns
+// over the rows of chunk y, 8 columns (16 bytes where aligned) x 32 rows at a
+// time, into P[y][col]; the second kernel sums the chunks. The loads of four
+// steps are in flight together. (A thread per column over 256 rows in turn, two
+// bytes per load, took 60 us for 32,768 x 256: 128 blocks of dependent loads.)
+__global__ void __launch_bounds__(256) colsum_bf16_kernel(const int M, const int N, const u16* __restrict__ X,
+                                                          const long ld, const int rowsPerChunk, const bool vec,
+                                                          float* __restrict__ P) {
+  __shared__ float s_a[32][65];
+  const int t = threadIdx.x, cg = t & 7, rl = t >> 3;
+  const int c0 = blockIdx.x * 64 + cg * 8;
+  const int r0 = blockIdx.y * rowsPerChunk, r1 = min(M, r0 + rowsPerChunk);
+  float a[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) a[j] = 0.f;
+  if (vec && c0 + 8 <= N) {
+    for (int r = r0 + rl; r < r1; r += 128) {
+      u32x4 w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = *reinterpret_cast<const u32x4*>(X + (long)min(r + 32 * u, r1 - 1) * ld + c0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (r + 32 * u < r1)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) a[j] += bf2f((u16)((j & 1) ? (w[u][j >> 1] >> 16) : (w[u][j >> 1] & 0xffffu)));
+    }
+  } else {
+    for (int r = r0 + rl; r < r1; r += 32)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (c0 + j < N) a[j] += bf2f(X[(long)r * ld + c0 + j]);
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) s_a[rl][cg * 8 + j] = a[j];
+  __syncthreads();
+  if (t < 64 && blockIdx.x * 64 + t < N) {
+    float v = 0.f;
+#pragma unroll
+    for (int r = 0; r < 32; ++r) v += s_a[r][t];
+    P[(long)blockIdx.y * N + blockIdx.x * 64 + t] = v;
   }
 }
-
-// partial column sums of a BF16 [M][ld] matrix: P[chunk][col]
-__global__ void __launch_bounds__(256) colsum_bf16_kernel(const int M, const int N, const u16* __restrict__ X,
-                                                          const long ld, const int rowsPerChunk,
-                                                          float* __restrict__ P) {
-  const int col = blockIdx.x * blockDim.x + threadIdx.x;
-  if (col >= N) return;
-  const int r0 = blockIdx.y * rowsPerChunk, r1 = min(M, r0 + rowsPerChunk);
-  float a = 0.f;
-  for (int r = r0; r < r1; ++r) a += bf2f(X[(long)r * ld + col]);
-  P[(long)blockIdx.y * N + col] = a;
+// The partial sums of a weight gradient, in one launch (two of their own cost a
+// launch each, ~4.7 us): blocks below sumBlocks form out[i] = sum_s P[s*n + i], s in
+// order (deterministic), with eight loads in flight (32 splits of 229,376 entries
+// took 30 us as a chain of dependent loads, 6 us so); the rest form 16 column sums
+// each from the C <= 128 chunks of Pc, eight per segment.
+__global__ void __launch_bounds__(256) weight_finish_kernel(const long n, const int S, const float* __restrict__ P,
+                                                            float* __restrict__ out, const int sumBlocks, const int N,
+                                                            const int C, const float* __restrict__ Pc,
+                                                            float* __restrict__ db) {
+  if (blockIdx.x < (unsigned)sumBlocks) {
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)sumBlocks * blockDim.x) {
+      float a = 0.f;
+      for (int s0 = 0; s0 < S; s0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = P[(long)min(s0 + u, S - 1) * n + i];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (s0 + u < S) a += v[u];
+      }
+      out[i] = a;
+    }
+    return;
+  }
+  __shared__ float s_a[16][17];
+  const int col = (blockIdx.x - sumBlocks) * 16 + (threadIdx.x & 15), seg = threadIdx.x >> 4;
+  float v[8], a = 0.f;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) v[u] = Pc[(long)min(seg + 16 * u, C - 1) * N + min(col, N - 1)];
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    if (seg + 16 * u < C) a += v[u];
+  s_a[seg][threadIdx.x & 15] = a;
+  __syncthreads();
+  if (seg == 0 && col < N) {
+    float b = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) b += s_a[k][threadIdx.x];
+    db[col] = b;
+  }
 }
 
 __global__ void __launch_bounds__(256) f32_to_bf16_kernel(const long n, const float* __restrict__ x,
@@ -266,14 +599,17 @@ __global__ void __launch_bounds__(256) adam_kernel(const int n, float* __restric
   }
 }
 
-// split-K sizing of the weight gradient (reduction over M rows)
-static void weight_splits(int M, int& S, int& kChunk) {
-  S = (M + 1023) / 1024;
+// Split-K sizing of the weight gradient (reduction over M rows): as many splits
+// as give two workgroups per CU over the output tiles, of 256 rows at least and
+// 64 splits at most, so that the partial sums stay few.
+static void weight_splits(int M, int K, int Nout, int& S, int& kChunk) {
+  const int tiles = ((K + GBN - 1) / GBN) * ((Nout + GBM - 1) / GBM);
+  S = (512 + tiles - 1) / tiles;
+  S = std::min(std::min(S, 64), (M + 255) / 256);
+  if (S >= 8) S = S / 8 * 8;
   if (S < 1) S = 1;
-  if (S > 64) S = 64;
   kChunk = ((M + S - 1) / S + GBK - 1) / GBK * GBK;
-  S = (M + kChunk - 1) / kChunk;
-  if (S < 1) S = 1;
+  if (S < 8) S = std::max(1, (M + kChunk - 1) / kChunk);  // from 8 on, trailing splits may be empty (zero partials)
 }
 static int colsum_chunks(int M) { return M < 256 ? 1 : (M + 255) / 256 > 128 ? 128 : (M + 255) / 256; }
 
@@ -314,7 +650,7 @@ extern "C" int libp_mlp_linear_bwd_data(int M, int K, int Nout, const unsigned s
 
 extern "C" long libp_mlp_ws_bytes(int M, int K, int Nout) {
   int S, kc;
-  weight_splits(M, S, kc);
+  weight_splits(M, K, Nout, S, kc);
   return (long)S * Nout * K * 4 + (long)colsum_chunks(M) * Nout * 4 + 256;
 }
 
@@ -325,26 +661,24 @@ extern "C" int libp_mlp_linear_bwd_weight(int M, int K, int Nout, const unsigned
   if (!dY || !X || !dWt || !ws) return arg_error("mlp_linear_bwd_weight", "null pointer");
   if (lddy < Nout || ldx < K) return arg_error("mlp_linear_bwd_weight", "leading dimension");
   int S, kc;
-  weight_splits(M, S, kc);
+  weight_splits(M, K, Nout, S, kc);
   float* P = reinterpret_cast<float*>(ws);
   // dWt[n][k] = sum_m dY[m][n] X[m][k]: A(n, m) = dY[m*lddy + n], B(k, m) = X[m*ldx + k] (both transposed)
   GemmArgs g{Nout, K, M, dY, lddy, X, ldx, P, K, nullptr, nullptr, 0, kc};
   int st = gemm<true, true, EPI_F32_PARTIAL>(g, S, stream, "mlp_linear_bwd_weight");
   if (st) return st;
   const long n = (long)Nout * K;
-  hipLaunchKernelGGL(sum_splits_kernel, dim3(stream_blocks(n, 256, 4096)), dim3(256), 0, as_stream(stream), n, S,
-                     P, dWt);
-  if ((st = launch_status("mlp_linear_bwd_weight"))) return st;
+  const unsigned sumBlocks = stream_blocks(n, 256, 4096);
+  const int C = colsum_chunks(M);
+  float* Pc = P + (long)S * Nout * K;
   if (db) {
-    const int C = colsum_chunks(M);
-    float* Pc = P + (long)S * Nout * K;
-    hipLaunchKernelGGL(colsum_bf16_kernel, dim3((Nout + 255) / 256, C), dim3(256), 0, as_stream(stream), M, Nout, dY,
-                       lddy, (M + C - 1) / C, Pc);
-    hipLaunchKernelGGL(sum_splits_kernel, dim3(stream_blocks(Nout, 256, 64)), dim3(256), 0, as_stream(stream),
-                       (long)Nout, C, Pc, db);
-    st = launch_status("mlp_linear_bwd_weight");
+    const bool vec = (lddy % 8) == 0 && ((uintptr_t)dY & 15) == 0;
+    hipLaunchKernelGGL(colsum_bf16_kernel, dim3((Nout + 63) / 64, C), dim3(256), 0, as_stream(stream), M, Nout, dY,
+                       lddy, (M + C - 1) / C, vec, Pc);
   }
-  return st;
+  hipLaunchKernelGGL(weight_finish_kernel, dim3(sumBlocks + (db ? (Nout + 15) / 16 : 0)), dim3(256), 0,
+                     as_stream(stream), n, S, P, dWt, (int)sumBlocks, Nout, C, Pc, db);
+  return launch_status("mlp_linear_bwd_weight");
 }
 
 extern "C" int libp_adam_step(int n, float* master, unsigned short* wbf16, const float* grad, float* m, float* v,

@@ -1,0 +1,66 @@
+"""The learned smoother's BF16 products at the edges of their tiles (128 x 128, 64 deep)
+and of the split sums: rows, columns and depths that are no multiple of a tile, with the
+vector accesses (contiguous dimension a multiple of 8) and without.
+
+Each FP32 sum of n products is within n 2^-24 of the sum of their magnitudes, in any
+order (products of two BF16 values are exact in FP32); a BF16 result adds half a BF16
+ulp, 2^-8 of the value.
+"""
+import pytest
+import torch
+
+import libparanumal_amd as lp
+
+pytestmark = pytest.mark.gpu
+
+
+def product(a, b):
+    """a @ b in FP64 and the bound of an FP32 sum of its depth."""
+    a, b = a.double(), b.double()
+    return a @ b, a.shape[1] * 2.0**-23 * (a.abs() @ b.abs()) + 1e-30
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 8, 8), (5, 72, 24), (127, 64, 128), (128, 128, 128), (257, 136, 264),
+                                   (257, 150, 130), (300, 7, 9), (2055, 64, 256), (4099, 264, 136), (16411, 72, 8)])
+def test_mlp_products_at_tile_edges(M, K, N):
+    L = lp.lib()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + K + N)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()  # noqa: E731
+    X, W, dY, H = rnd(M, K), rnd(N, K), rnd(M, N), rnd(M, K)
+    b, scale = torch.randn(N, device="cuda", generator=g), torch.rand(M, device="cuda", generator=g) + 0.5
+    st = torch.cuda.current_stream().cuda_stream
+    nan = float("nan")
+    ref, bound = product(X, W.T)
+    bound = bound + 2.0**-22 * (ref.abs() + b.double().abs())
+    Y = torch.full((M, N), nan, device="cuda")
+    lp.check(L.libp_mlp_linear_fwd(M, K, N, X.data_ptr(), K, W.data_ptr(), K, b.data_ptr(), 0, Y.data_ptr(), N, st))
+    Ys = torch.full((M, N), nan, device="cuda")
+    lp.check(L.libp_mlp_linear_fwd_scaled(M, K, N, X.data_ptr(), K, W.data_ptr(), K, None, scale.data_ptr(),
+                                          Ys.data_ptr(), N, st))
+    Yr = torch.full((M, N), nan, device="cuda").bfloat16()
+    lp.check(L.libp_mlp_linear_fwd(M, K, N, X.data_ptr(), K, W.data_ptr(), K, b.data_ptr(), 1, Yr.data_ptr(), N, st))
+    torch.cuda.synchronize()
+    assert ((Y.double() - (ref + b.double())).abs() <= bound).all()
+    assert ((Ys.double() - scale.double()[:, None] * ref).abs() <= 2 * bound).all()
+    relu = torch.relu(ref + b.double())
+    assert ((Yr.double() - relu).abs() <= bound + 2.0**-8 * relu).all()
+
+    ref, bound = product(dY, W)
+    for mask in (None, H):
+        dX = torch.full((M, K), nan, device="cuda").bfloat16()
+        lp.check(L.libp_mlp_linear_bwd_data(M, K, N, dY.data_ptr(), N, W.data_ptr(), K,
+                                            mask.data_ptr() if mask is not None else None, K, dX.data_ptr(), K, st))
+        torch.cuda.synchronize()
+        want = ref if mask is None else torch.where(H.double() > 0, ref, 0.0)
+        assert ((dX.double() - want).abs() <= bound + 2.0**-8 * want.abs()).all()
+
+    dW, db = torch.full((N, K), nan, device="cuda"), torch.full((N,), nan, device="cuda")
+    ws = torch.full((L.libp_mlp_ws_bytes(M, K, N) // 4,), nan, device="cuda")
+    lp.check(L.libp_mlp_linear_bwd_weight(M, K, N, dY.data_ptr(), N, X.data_ptr(), K, dW.data_ptr(), db.data_ptr(),
+                                          ws.data_ptr(), st))
+    torch.cuda.synchronize()
+    ref, bound = product(dY.T, X)
+    assert ((dW.double() - ref).abs() <= bound).all()
+    mag = dY.double().abs().sum(0)
+    assert ((db.double() - dY.double().sum(0)).abs() <= M * 2.0**-23 * mag).all()
