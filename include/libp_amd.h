@@ -270,6 +270,26 @@ long libp_pcg_gather_jacobi_partials(int Nrows);
 int libp_pcg_gather_jacobi_update_f64(int Nrows, const int* rowStarts, const int* colIds, const double* AqL,
                                       const double* invDiag, const double* p, double* x, double* r, double* z,
                                       double* scalars, double* partials, void* stream);
+/* One whole Jacobi-PCG iteration in three launches, for problems small enough that
+ * the launches which sum partials dominate (libp_pcg_jacobi_iteration_folds: at most
+ * 1024 partial sums of the Ax and of the gather): the p update, the Ax with p.Ap and
+ * the gather with the x, r, z update, where each kernel forms the sums of the one
+ * before it by itself. p, x, r, z and the scalars are those of libp_pcg_update_p_f64,
+ * libp_pcg_ax_hex_pap_f64 and libp_pcg_gather_jacobi_update_f64, bit for bit.
+ * states holds two blocks of 16 doubles in the layout of the scalars, zeroed before
+ * the first iteration (it = 0) except states[16 + RDOTZ1] = r.z (libp_pcg_jacobi_rdotz_f64
+ * with scalars = states + 16) and states[16 + TOL]; iteration it leaves its scalars in
+ * block it & 1 and does nothing once STOP is set. papPartials and gatherPartials are
+ * sized as for the two calls. _check writes the scalars after iteration it (RDOTZ1, RDOTR,
+ * TOL, STOP, ITERS) into pinned host memory mapped for the device. */
+int libp_pcg_jacobi_iteration_folds(int N, int Nelements, int Nrows);
+int libp_pcg_jacobi_iteration_f64(int N, int Nelements, const int* elementList, const int* GlobalToLocal,
+                                  const double* wJ, const double* ggeo, const double* D, double lambda, int Nrows,
+                                  const int* rowStarts, const int* colIds, const double* invDiag, int it, double* p,
+                                  double* AqL, double* x, double* r, double* z, double* papPartials,
+                                  double* gatherPartials, double* states, void* stream);
+int libp_pcg_jacobi_iteration_check_f64(int Nrows, int it, const double* states, const double* gatherPartials,
+                                        double* hostScalars, void* stream);
 /* scalars[TOL] = tol^2 * scalars[RDOTR] (1e-300 when that is 0), and
  * scalars[STOP] = 1 when scalars[RDOTR] is 0: the pure relative stopping rule
  * of a solve from a zero guess, formed on the device instead of after a host

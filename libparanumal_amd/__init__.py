@@ -126,6 +126,10 @@ SIGNATURES = {
     "libp_nbfpcg_update0_f64": (c_int, [c_int] + [c_void_p] * 6),
     "libp_nbfpcg_update1_f64": (c_int, [c_int] + [c_void_p] * 11),
     "libp_nbfpcg_update2_f64": (c_int, [c_int] + [c_void_p] * 10),
+    "libp_pcg_jacobi_iteration_folds": (c_int, [c_int, c_int, c_int]),
+    "libp_pcg_jacobi_iteration_f64": (c_int, [c_int, c_int] + [c_void_p] * 5 + [c_double, c_int] + [c_void_p] * 3 +
+                                      [c_int] + [c_void_p] * 9),
+    "libp_pcg_jacobi_iteration_check_f64": (c_int, [c_int, c_int] + [c_void_p] * 4),
     "libp_mlp_linear_fwd": (c_int, [c_int, c_int, c_int, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int,
                                     c_void_p, c_long, c_void_p]),
     "libp_mlp_linear_fwd_scaled": (c_int, [c_int, c_int, c_int, c_void_p, c_long, c_void_p, c_long, c_void_p,

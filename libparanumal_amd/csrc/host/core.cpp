@@ -208,15 +208,18 @@ platform_t::platform_t(const settings_t& s) {
   hipStream_t st;
   LIBP_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
   double* pinned = nullptr;
-  LIBP_HIP(hipHostMalloc((void**)&pinned, 16 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
+  LIBP_HIP(hipHostMalloc((void**)&pinned, 48 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
   hipEvent_t ev = nullptr;
   LIBP_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   struct State {
     hipStream_t st = nullptr;
     double* pinned = nullptr;
-    hipEvent_t ev = nullptr;
+    hipEvent_t ev = nullptr, pipe[2] = {nullptr, nullptr};
     ~State() {
+      if (st) (void)hipStreamSynchronize(st);  // a queued check may still write the pinned scalars
       if (ev) (void)hipEventDestroy(ev);
+      for (hipEvent_t e : pipe)
+        if (e) (void)hipEventDestroy(e);
       if (st) (void)hipStreamDestroy(st);
       if (pinned) (void)hipHostFree(pinned);
     }
@@ -230,6 +233,12 @@ platform_t::platform_t(const settings_t& s) {
   h_scalars = pinned;
   ev_read = ev;
   LIBP_HIP(hipHostGetDevicePointer((void**)&d_hScalars, pinned, 0));
+  for (int k = 0; k < 2; ++k) {
+    LIBP_HIP(hipEventCreateWithFlags(&stt->pipe[k], hipEventDisableTiming));
+    ev_pipe[k] = stt->pipe[k];
+    h_pipe[k] = pinned + 16 * (k + 1);
+    d_pipe[k] = d_hScalars + 16 * (k + 1);
+  }
   o_reduceWS = deviceMemory<char>::alloc((size_t)libp_reduce_ws_bytes());
   LIBP_HIP(hipMemsetAsync(o_reduceWS.ptr(), 0, o_reduceWS.length(), stream));
   o_scalars = deviceMemory<double>::alloc(64);

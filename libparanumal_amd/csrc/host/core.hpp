@@ -183,6 +183,11 @@ class platform_t {
   double* h_scalars = nullptr;     // pinned mirror (16 doubles), mapped for the device
   double* d_hScalars = nullptr;    // its device pointer
   hipEvent_t ev_read = nullptr;    // recorded behind each read
+  // two more pinned blocks of 16 scalars (host and device pointers) and their events,
+  // for a solver that queues its next chunk before it waits for the last one's scalars
+  double* h_pipe[2] = {nullptr, nullptr};
+  double* d_pipe[2] = {nullptr, nullptr};
+  hipEvent_t ev_pipe[2] = {nullptr, nullptr};
 
   platform_t() {}
   explicit platform_t(const settings_t& s);

@@ -30,10 +30,7 @@ void elliptic_t::SetupPrecon() {
     precon.Setup<JacobiPrecon>(*this);
     // the fused Jacobi-PCG iteration's reduction partials, allocated here rather
     // than inside a timed solve
-    if (settings.compareSetting("PCG FUSED OPERATOR", "TRUE") && mesh.N >= 1 && mesh.N <= 15) {
-      o_axPartials = platform.malloc<double>(std::max(libp_ax_hex_split_blocks(mesh.N, mesh.NlocalGatherElements), 1));
-      o_gatherPartials = platform.malloc<double>(std::max<long>(libp_pcg_gather_jacobi_partials(ogsMasked.NlocalT), 2));
-    }
+    if (settings.compareSetting("PCG FUSED OPERATOR", "TRUE") && mesh.N >= 1 && mesh.N <= 15) jacobiPCGPartials();
   } else if (settings.compareSetting("PRECONDITIONER", "MULTIGRID")) {
     precon.Setup<MultiGridPrecon>(*this);
   } else if (settings.compareSetting("PRECONDITIONER", "NONE")) {
@@ -191,15 +188,41 @@ void elliptic_t::Operator(deviceMemory<dfloat>& o_q, deviceMemory<dfloat>& o_Aq)
   ogsMasked.Gather(o_Aq, o_AqL, 1, ogs::Add, ogs::Trans);
 }
 
+void elliptic_t::jacobiPCGPartials() {
+  if (o_gatherPartials.isInitialized()) return;
+  o_axPartials = platform.malloc<double>(std::max(libp_ax_hex_split_blocks(mesh.N, mesh.NlocalGatherElements), 1));
+  o_gatherPartials = platform.malloc<double>(std::max<long>(libp_pcg_gather_jacobi_partials(ogsMasked.NlocalT), 2));
+}
+
+bool elliptic_t::hasJacobiPCGIteration() {
+  if (!settings.compareSetting("PCG FUSED OPERATOR", "TRUE") || mesh.N < 1 || mesh.N > 15 || SplitGather() ||
+      !libp_pcg_jacobi_iteration_folds(mesh.N, mesh.NlocalGatherElements, ogsMasked.NlocalT))
+    return false;
+  jacobiPCGPartials();
+  return true;
+}
+
+void elliptic_t::JacobiPCGIteration(int it, deviceMemory<dfloat>& o_p, deviceMemory<dfloat>& o_x,
+                                    deviceMemory<dfloat>& o_r, deviceMemory<dfloat>& o_z,
+                                    const deviceMemory<dfloat>& o_invDiag, double* states) {
+  LIBP_CALL(libp_pcg_jacobi_iteration_f64(
+      mesh.N, mesh.NlocalGatherElements, nullptr, o_GlobalToLocal.ptr(), mesh.o_wJ.ptr(), mesh.o_ggeo.ptr(),
+      mesh.o_D.ptr(), lambda, ogsMasked.NlocalT, ogsMasked.o_rowStartsT.ptr(), ogsMasked.o_colIdsT.ptr(),
+      o_invDiag.ptr(), it, o_p.ptr(), o_AqL.ptr(), o_x.ptr(), o_r.ptr(), o_z.ptr(), o_axPartials.ptr(),
+      o_gatherPartials.ptr(), states, platform.s()));
+}
+
+void elliptic_t::jacobiPCGCheck(int it, const double* states, double* hostScalars) {
+  LIBP_CALL(libp_pcg_jacobi_iteration_check_f64(ogsMasked.NlocalT, it, states, o_gatherPartials.ptr(), hostScalars,
+                                                platform.s()));
+}
+
 bool elliptic_t::OperatorJacobiPCG(deviceMemory<dfloat>& o_p, deviceMemory<dfloat>& o_x, deviceMemory<dfloat>& o_r,
                                    deviceMemory<dfloat>& o_z, const deviceMemory<dfloat>& o_invDiag,
                                    double* scalars) {
   if (!settings.compareSetting("PCG FUSED OPERATOR", "TRUE") || mesh.N < 1 || mesh.N > 15 || SplitGather())
     return false;
-  if (!o_gatherPartials.isInitialized()) {
-    o_axPartials = platform.malloc<double>(std::max(libp_ax_hex_split_blocks(mesh.N, mesh.NlocalGatherElements), 1));
-    o_gatherPartials = platform.malloc<double>(std::max<long>(libp_pcg_gather_jacobi_partials(ogsMasked.NlocalT), 2));
-  }
+  jacobiPCGPartials();
   LIBP_CALL(libp_pcg_ax_hex_pap_f64(mesh.N, mesh.NlocalGatherElements, nullptr, o_GlobalToLocal.ptr(),
                                     mesh.o_wJ.ptr(), mesh.o_ggeo.ptr(), mesh.o_D.ptr(), lambda, o_p.ptr(),
                                     o_AqL.ptr(), o_axPartials.ptr(), scalars, platform.s()));
@@ -283,6 +306,8 @@ elliptic_t elliptic_t::SetupNewDegree(mesh_t& meshC) {
   if (meshC.N == mesh.N) return *this;
   elliptic_t e = *this;
   e.mesh = meshC;
+  e.o_axPartials = deviceMemory<double>();  // sized for this degree
+  e.o_gatherPartials = deviceMemory<double>();
   e.BoundarySetup();
   e.precon = precon_t();
   return e;

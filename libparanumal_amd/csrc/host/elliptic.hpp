@@ -93,7 +93,12 @@ class elliptic_t : public operator_t {
   // ([PCG FUSED OPERATOR] TRUE, N <= 15, two-pass operator; N = 15 on the MFMA kernel)
   bool OperatorJacobiPCG(deviceMemory<dfloat>& o_p, deviceMemory<dfloat>& o_x, deviceMemory<dfloat>& o_r,
                          deviceMemory<dfloat>& o_z, const deviceMemory<dfloat>& o_invDiag, double* scalars) override;
+  bool hasJacobiPCGIteration() override;
+  void JacobiPCGIteration(int it, deviceMemory<dfloat>& o_p, deviceMemory<dfloat>& o_x, deviceMemory<dfloat>& o_r,
+                          deviceMemory<dfloat>& o_z, const deviceMemory<dfloat>& o_invDiag, double* states) override;
+  void jacobiPCGCheck(int it, const double* states, double* hostScalars) override;
   deviceMemory<double> o_axPartials, o_gatherPartials;
+  void jacobiPCGPartials();  // allocates them
   void PartialAx(deviceMemory<dfloat>& o_q, deviceMemory<dfloat>& o_AqL);
   // the split operator's maps, or null when the two-pass form is used
   splitGather_t* SplitGather();

@@ -37,6 +37,27 @@ class operator_t {
     (void)scalars;
     return false;
   }
+  // A whole Jacobi-PCG iteration in three launches on two blocks of scalars
+  // (libp_pcg_jacobi_iteration_f64), for problems small enough; jacobiPCGCheck
+  // writes the scalars after iteration it to mapped host memory.
+  // hasJacobiPCGIteration is false when the operator or its size has no such form.
+  virtual bool hasJacobiPCGIteration() { return false; }
+  virtual void JacobiPCGIteration(int it, deviceMemory<dfloat>& o_p, deviceMemory<dfloat>& o_x,
+                                  deviceMemory<dfloat>& o_r, deviceMemory<dfloat>& o_z,
+                                  const deviceMemory<dfloat>& o_invDiag, double* states) {
+    (void)it;
+    (void)o_p;
+    (void)o_x;
+    (void)o_r;
+    (void)o_z;
+    (void)o_invDiag;
+    (void)states;
+  }
+  virtual void jacobiPCGCheck(int it, const double* states, double* hostScalars) {
+    (void)it;
+    (void)states;
+    (void)hostScalars;
+  }
   // For a preconditioner: z = M r together with the PCG scalars of
   // libp_pcg_rdotz_f64 (r.z, and z.Ap when flexible) in one pass over z.
   // Returns false when there is no fused form.
@@ -166,7 +187,10 @@ class pcg : public linearSolverBase_t {
   bool flexible = false;
   bool fuseJacobi = true;  // [PCG JACOBI FUSED]: p.Ap in the gather; fused Jacobi-PCG iterations
   deviceMemory<dfloat> o_p, o_z, o_Ax, o_Ap;
-  deviceMemory<dfloat> o_s;  // LIBP_PCG_NSCALARS device scalars
+  deviceMemory<dfloat> o_s;       // LIBP_PCG_NSCALARS device scalars
+  deviceMemory<dfloat> o_states;  // the two blocks of scalars of solveFolded
+  int solveFolded(operator_t& A, diagonalPrecon_t& jac, deviceMemory<dfloat>& o_x, deviceMemory<dfloat>& o_r,
+                  dfloat TOL, int MAXIT);
   void iteration(operator_t& linearOperator, operator_t& precon, diagonalPrecon_t* jac, int it,
                  deviceMemory<dfloat>& o_x, deviceMemory<dfloat>& o_r);
 

@@ -716,3 +716,58 @@ extern "C" int libp_pcg_ax_hex_pap_f64(int N, int Nelements, const int* elementL
       return arg_error("pcg_ax_hex_pap", "polynomial degree must be in [1,15]");
   }
 }
+
+namespace libp_amd {
+unsigned gather_jacobi_blocks(int Nrows);  // ogs.hip
+int launch_gather_jacobi_fold(int Nrows, const int* rowStarts, const int* colIds, const double* AqL,
+                              const double* invDiag, const double* p, double* x, double* r, double* z,
+                              const double* s, double* part, int nbAx, const double* papPart, hipStream_t st);
+int launch_update_p_fold(int N, int first, const double* z, double* p, const double* prev, double* cur, int nb,
+                         const double* part, hipStream_t st);  // linalg.hip
+}  // namespace libp_amd
+
+extern "C" int libp_pcg_jacobi_iteration_folds(int N, int Nelements, int Nrows) {
+  const int nbAx = libp_ax_hex_split_blocks(N, Nelements);
+  return Nelements > 0 && Nrows > 0 && nbAx > 0 && nbAx <= PCG_FOLD_MAX && gather_jacobi_blocks(Nrows) <= PCG_FOLD_MAX;
+}
+
+// Three launches per iteration: each sum of partials is formed by the kernel that needs it.
+// Small solves are bound by the latency of their launches (8^3 elements, N = 4: 2.8 + 5.1 +
+// 3.4 + 6.1 + 3.5 us in five; 3.9 + 4.8 + 6.5 us in three). PCG_FOLD_MAX partials are what
+// a block of 256 threads sums with four loads each; past it (16^3 elements at N = 4,
+// 524,288 rows) the finishers' 7 us are a small share of an iteration and every block
+// would read more than 8 KB of partials.
+extern "C" int libp_pcg_jacobi_iteration_f64(int N, int Nelements, const int* elementList, const int* GlobalToLocal,
+                                             const double* wJ, const double* ggeo, const double* D, double lambda,
+                                             int Nrows, const int* rowStarts, const int* colIds,
+                                             const double* invDiag, int it, double* p, double* AqL, double* x,
+                                             double* r, double* z, double* papPartials, double* gatherPartials,
+                                             double* states, void* stream) {
+  if (!GlobalToLocal || !wJ || !ggeo || !D || !rowStarts || !colIds || !invDiag || !p || !AqL || !x || !r || !z ||
+      !papPartials || !gatherPartials || !states || it < 0)
+    return arg_error("pcg_jacobi_iteration", "null pointer or negative iteration");
+  if (((uintptr_t)z & 15) || ((uintptr_t)p & 15)) return arg_error("pcg_jacobi_iteration", "p and z must be 16-byte aligned");
+  if (!libp_pcg_jacobi_iteration_folds(N, Nelements, Nrows))
+    return arg_error("pcg_jacobi_iteration", "degree out of range or too many partial sums");
+  hipStream_t st = as_stream(stream);
+  double* cur = states + 16 * (it & 1);
+  int rc = launch_update_p_fold(Nrows, it == 0, z, p, states + 16 * ((it + 1) & 1), cur,
+                                (int)gather_jacobi_blocks(Nrows), gatherPartials, st);
+  if (rc != LIBP_OK) return rc;
+  const AxArgs<double> a{Nelements, elementList, GlobalToLocal, wJ, ggeo, D, lambda, p, AqL, nullptr, papPartials,
+                         nullptr, cur, st};
+  switch (N) {
+#define LIBP_AX_CASE(NN)                                                   \
+  case NN:                                                                 \
+    rc = launch_ax<NN + 1, double, 0, 0, true>(a, "pcg_jacobi_iteration"); \
+    break;
+    LIBP_AX_CASES_1_14
+#undef LIBP_AX_CASE
+    default:
+      rc = launch_ax_mfma_n15_pap(Nelements, elementList, GlobalToLocal, wJ, ggeo, D, lambda, p, AqL, papPartials, cur,
+                                  st);
+  }
+  if (rc != LIBP_OK) return rc;
+  return launch_gather_jacobi_fold(Nrows, rowStarts, colIds, AqL, invDiag, p, x, r, z, cur, gatherPartials,
+                                   libp_ax_hex_split_blocks(N, Nelements), papPartials, st);
+}

@@ -385,6 +385,94 @@ __global__ void __launch_bounds__(256) pcg_update_p2_kernel(const int N, const i
   }
 }
 
+// The p update of a folded Jacobi-PCG iteration. Each block forms r.r and r.z of the
+// previous iteration from its nb <= PCG_FOLD_MAX pairs of partials (bit for bit the sums
+// of pcg_gather_jacobi_finish_kernel), the stopping test and beta itself; block 0 leaves
+// the iteration's scalars in cur, which this launch's other blocks do not read (they read
+// prev, which nobody writes: the two alternate). first: r.z is prev[RDOTZ1], beta = 0.
+__global__ void __launch_bounds__(256) pcg_update_p_fold_kernel(const int N, const int first,
+                                                                const double* __restrict__ z, double* __restrict__ p,
+                                                                const double* __restrict__ prev,
+                                                                double* __restrict__ cur, const int nb,
+                                                                const double* __restrict__ part) {
+  __shared__ double s_w[16];
+  const long N2 = N / 2;
+  const pcg_v2d* z2 = (const pcg_v2d*)z;
+  pcg_v2d* p2 = (pcg_v2d*)p;
+  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+  pcg_v2d zv = {0.0, 0.0}, pv = {0.0, 0.0};
+  if (N2 > 0) {  // loaded beside the partials (clamped: the last block's spare threads)
+    zv = z2[i < N2 ? i : N2 - 1];
+    pv = p2[i < N2 ? i : N2 - 1];
+  }
+  double rz = prev[0], rr = prev[5], iters = prev[9], beta = 0.0;
+  const double tol = prev[7];
+  bool stop = prev[8] != 0.0;
+  if (!first && !stop) {
+    const FoldedSum f0 = folded_load(part, nb), f1 = folded_load(part + nb, nb);
+    rr = folded_sum(f0, s_w);
+    const double rzn = folded_sum(f1, s_w);
+    beta = rzn / rz;
+    rz = rzn;
+    iters += 1.0;
+    stop = tol > 0.0 && rr <= tol;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    cur[0] = rz;
+    cur[1] = prev[0];
+    cur[3] = beta;
+    cur[5] = rr;
+    cur[7] = tol;
+    cur[8] = stop ? 1.0 : 0.0;
+    cur[9] = iters;
+  }
+  if (stop) return;
+  if (i < N2) {
+    pcg_v2d o;
+    if (beta != 0)
+      o = 1.0 * zv + beta * pv;
+    else
+      o = 1.0 * zv;
+    p2[i] = o;
+  }
+  if ((N & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+    const int n = N - 1;
+    p[n] = (beta != 0) ? 1.0 * z[n] + beta * p[n] : 1.0 * z[n];
+  }
+}
+
+// The scalars after a folded iteration, as pcg_gather_jacobi_finish_kernel would leave
+// them, into pinned host memory mapped for the device (the next iteration's p update
+// forms the same sums again; nothing on the device changes here).
+__global__ void __launch_bounds__(256) pcg_fold_check_kernel(const int nb, const double* __restrict__ cur,
+                                                             const double* __restrict__ part,
+                                                             double* __restrict__ host) {
+  __shared__ double s_w[16];
+  double rz = cur[0], rr = cur[5], iters = cur[9];
+  bool stop = cur[8] != 0.0;
+  if (!stop) {
+    const FoldedSum f0 = folded_load(part, nb), f1 = folded_load(part + nb, nb);
+    rr = folded_sum(f0, s_w);
+    rz = folded_sum(f1, s_w);
+    iters += 1.0;
+    stop = cur[7] > 0.0 && rr <= cur[7];
+  }
+  if (threadIdx.x == 0) {
+    host[0] = rz;
+    host[5] = rr;
+    host[7] = cur[7];
+    host[8] = stop ? 1.0 : 0.0;
+    host[9] = iters;
+  }
+}
+
+int launch_update_p_fold(int N, int first, const double* z, double* p, const double* prev, double* cur, int nb,
+                         const double* part, hipStream_t st) {
+  hipLaunchKernelGGL(pcg_update_p_fold_kernel, dim3((N / 2 + 255) / 256 + (N < 2)), dim3(256), 0, st, N, first, z, p,
+                     prev, cur, nb, part);
+  return launch_status("pcg_jacobi_iteration");
+}
+
 __global__ void __launch_bounds__(RBS) pcg_jacobi_update_kernel(const int N, const double* __restrict__ invDiag,
                                                                 const double* __restrict__ p,
                                                                 const double* __restrict__ Ap,
@@ -744,4 +832,18 @@ extern "C" int libp_hbm_probe_f64(int mode, long n, const double* x, double* y, 
     return arg_error("hbm_probe", "mode must be 0 (read) or 1 (copy)");
   }
   return launch_status("hbm_probe");
+}
+
+namespace libp_amd {
+unsigned gather_jacobi_blocks(int Nrows);  // ogs.hip
+}
+extern "C" int libp_pcg_jacobi_iteration_check_f64(int Nrows, int it, const double* states,
+                                                   const double* gatherPartials, double* hostScalars, void* stream) {
+  if (!states || !gatherPartials || !hostScalars || it < 0 || Nrows <= 0)
+    return arg_error("pcg_jacobi_iteration_check", "null pointer or bad size");
+  const unsigned nb = gather_jacobi_blocks(Nrows);
+  if (nb > PCG_FOLD_MAX) return arg_error("pcg_jacobi_iteration_check", "too many rows");
+  hipLaunchKernelGGL(pcg_fold_check_kernel, dim3(1), dim3(256), 0, as_stream(stream), (int)nb, states + 16 * (it & 1),
+                     gatherPartials, hostScalars);
+  return launch_status("pcg_jacobi_iteration_check");
 }

@@ -284,10 +284,14 @@ inline unsigned face_gather_blocks(int Nrows) { return stream_blocks(Nrows, 1024
 // the gathered E-vector were slower (605 us): neighbouring row blocks share its
 // cache lines.
 constexpr long GATHER_JACOBI_MAXB = 1L << 20;
-inline unsigned gather_jacobi_blocks(int Nrows) {
+unsigned gather_jacobi_blocks(int Nrows) {
   return (unsigned)std::max<long>(1, std::min<long>(gather_row_blocks(Nrows), GATHER_JACOBI_MAXB));
 }
 
+// FOLD: s[ALPHA] has not been formed; each block forms p.Ap from the Ax kernel's nbAx <=
+// PCG_FOLD_MAX partials itself (loaded ahead of the gather, in its shadow) and alpha =
+// s[RDOTZ1] / p.Ap, the same to the bit, so no finisher runs in between.
+template <bool FOLD>
 __global__ void __launch_bounds__(GB_THREADS) pcg_gather_jacobi_kernel(const int Nrows,
                                                                        const int* __restrict__ rowStarts,
                                                                        const int* __restrict__ colIds,
@@ -298,11 +302,14 @@ __global__ void __launch_bounds__(GB_THREADS) pcg_gather_jacobi_kernel(const int
                                                                        double* __restrict__ r,
                                                                        double* __restrict__ z,
                                                                        const double* __restrict__ s,
-                                                                       double* __restrict__ part) {
+                                                                       double* __restrict__ part, const int nbAx,
+                                                                       const double* __restrict__ papPart) {
   __shared__ double s_v[GB_CAP];
   __shared__ double s_w[16];
   if (s[8] != 0.0) return;
-  const double alpha = s[2];
+  double alpha = FOLD ? s[0] : s[2];
+  FoldedSum pap;
+  if (FOLD) pap = folded_load(papPart, nbAx);
   const long nrb = gather_row_blocks(Nrows);
   double a0 = 0, a1 = 0;
   for (long rb = blockIdx.x; rb < nrb; rb += gridDim.x) {
@@ -318,6 +325,7 @@ __global__ void __launch_bounds__(GB_THREADS) pcg_gather_jacobi_kernel(const int
     }
     GatherRows<double> g;
     gather_block_sums(rb, Nrows, rowStarts, colIds, v, s_v, g);
+    if (FOLD) alpha = s[0] / folded_sum(pap, s_w);
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       if (!g.in[u]) continue;
@@ -382,6 +390,15 @@ __global__ void __launch_bounds__(1024) pcg_gather_jacobi_finish_kernel(const in
     s[0] = rz;
     s[3] = rz / s[1];
   }
+}
+
+// The gather-update of a folded iteration (ax_hex.hip): alpha from the Ax partials.
+int launch_gather_jacobi_fold(int Nrows, const int* rowStarts, const int* colIds, const double* AqL,
+                              const double* invDiag, const double* p, double* x, double* r, double* z,
+                              const double* s, double* part, int nbAx, const double* papPart, hipStream_t st) {
+  hipLaunchKernelGGL(pcg_gather_jacobi_kernel<true>, dim3(gather_jacobi_blocks(Nrows)), dim3(GB_THREADS), 0, st, Nrows,
+                     rowStarts, colIds, AqL, invDiag, p, x, r, z, s, part, nbAx, papPart);
+  return launch_status("pcg_jacobi_iteration");
 }
 
 template <typename T>
@@ -535,8 +552,9 @@ extern "C" int libp_pcg_gather_jacobi_update_f64(int Nrows, const int* rowStarts
   if (!rowStarts || !colIds || !AqL || !invDiag || !p || !x || !r || !z || !scalars || !partials)
     return arg_error("pcg_gather_jacobi_update", "null pointer");
   const unsigned nb = gather_jacobi_blocks(Nrows);
-  hipLaunchKernelGGL(pcg_gather_jacobi_kernel, dim3(nb), dim3(GB_THREADS), 0, as_stream(stream), Nrows, rowStarts,
-                     colIds, AqL, invDiag, p, x, r, z, (const double*)scalars, partials);
+  hipLaunchKernelGGL(pcg_gather_jacobi_kernel<false>, dim3(nb), dim3(GB_THREADS), 0, as_stream(stream), Nrows,
+                     rowStarts, colIds, AqL, invDiag, p, x, r, z, (const double*)scalars, partials, 0,
+                     (const double*)nullptr);
   const int nb1 = gather_jacobi_stage1_blocks(nb);
   if (nb1 > 0) {
     double* sums = partials + 2L * nb;

@@ -70,6 +70,41 @@ __device__ inline double strided_sum(const double* __restrict__ x, const int n) 
   return t;
 }
 
+// The same sum as block_sum(strided_sum(x, n)) of a 1024-thread block, bit for bit, for
+// n <= PCG_FOLD_MAX, formed by a 256-thread block and known to every thread: each wavefront
+// sums four of the sixteen groups of 64 entries. A kernel that starts with it needs no
+// finisher launch before it; the loads can be issued (folded_load) ahead of the kernel's own.
+constexpr int PCG_FOLD_MAX = 1024;
+struct FoldedSum {
+  double v[4];
+  int n;
+};
+__device__ inline FoldedSum folded_load(const double* __restrict__ x, const int n) {
+  FoldedSum f;
+  f.n = n;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int i = ((threadIdx.x >> 6) + 4 * u) * 64 + (threadIdx.x & 63);
+    const double v = x[min(i, n - 1)];
+    f.v[u] = i < n ? 0.0 + v : 0.0;
+  }
+  return f;
+}
+__device__ inline double folded_sum(const FoldedSum& f, double* s_w) {  // s_w: 16 entries
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int w = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) + 4 * u);
+    const double g = w * 64 < f.n ? wave_sum(f.v[u]) : 0.0;  // a group past the end sums to 0
+    if ((threadIdx.x & 63) == 0) s_w[w] = g;
+  }
+  __syncthreads();
+  double r = 0;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r += s_w[i];
+  __syncthreads();
+  return r;
+}
+
 // One partial per block for each of NV sums: ws->part[k][blockIdx.x].
 template <int NV>
 __device__ inline void store_block_partials(ReduceWS* ws, const double (&v)[NV], double* s_w) {
