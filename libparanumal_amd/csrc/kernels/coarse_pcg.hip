@@ -535,8 +535,22 @@ __global__ void __launch_bounds__(64) coarse_cg1_check_kernel(const int nb, doub
 // partials of the previous launch are read from wsIn and this launch's are
 // written to wsOut, a different workspace: the blocks of one launch need not
 // all be resident at once, so one block may finish before another starts.
-constexpr int CSR_THREADS = 1024, CSR_LANES = 8, CSR_ROWS = CSR_THREADS / CSR_LANES, CSR_UNROLL = 32 / CSR_LANES;
+constexpr int CSR_LANES = 8, CSR_UNROLL = 32 / CSR_LANES;
 
+// Threads per block: few blocks keep the partial sums that every block reads few (at
+// 29,791 rows, 233 blocks of 1024 threads beat 466 of 512 and 932 of 256), but below 256
+// blocks CUs are left idle while the others issue more of the divergent column loads:
+// the smallest block that gives at most 256 of them. 4,845 rows: 38 blocks of 1024 threads
+// took 9.2 us per iteration, 152 of 256 take 6.8 us (the three block sums behind one barrier).
+static int csr_threads(int Nrows) {
+  return Nrows <= 256 * (256 / CSR_LANES) ? 256 : Nrows <= 256 * (512 / CSR_LANES) ? 512 : 1024;
+}
+static int csr_blocks(int Nrows) {
+  const int rows = csr_threads(Nrows) / CSR_LANES;
+  return std::min((Nrows + rows - 1) / rows, RMAXB);
+}
+
+template <int CSR_THREADS>
 __global__ void __launch_bounds__(CSR_THREADS) coarse_cg1_csr_kernel(
     const int Nrows, const int* __restrict__ rowStarts, const int* __restrict__ colIds,
     const double* __restrict__ vals, const int mode, const int P, const double tol2, const int nb,
@@ -544,9 +558,10 @@ __global__ void __launch_bounds__(CSR_THREADS) coarse_cg1_csr_kernel(
     double* __restrict__ wcur, double* __restrict__ wnxt, double* s, const ReduceWS* __restrict__ wsIn,
     ReduceWS* __restrict__ wsOut) {
 #pragma clang fp contract(off)
+  constexpr int CSR_ROWS = CSR_THREADS / CSR_LANES;
   __shared__ double s_ab[2];
   __shared__ int s_stop;
-  __shared__ double s_w[16];
+  __shared__ double s_w[3][16];
   // u at gathered dof j after this iteration's update, from its loaded
   // r, w, s and invD
   auto unew = [&](double ro, double wo, double so, double dg, double alpha, double beta) -> double {
@@ -651,13 +666,17 @@ __global__ void __launch_bounds__(CSR_THREADS) coarse_cg1_csr_kernel(
       }
     }
   }
-  const double b0 = block_sum(ga, s_w);
-  const double b1 = block_sum(de, s_w);
-  const double b2 = block_sum(rr, s_w);
-  if (threadIdx.x == 0) {
-    wsOut->part[0][blockIdx.x] = b0;
-    wsOut->part[1][blockIdx.x] = b1;
-    wsOut->part[2][blockIdx.x] = b2;
+  // the three block sums behind one barrier, each in the order of block_sum
+  const double sums[3] = {wave_sum(ga), wave_sum(de), wave_sum(rr)};
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) s_w[k][threadIdx.x >> 6] = sums[k];
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    double t = 0;
+#pragma unroll
+    for (int i = 0; i < CSR_THREADS / 64; ++i) t += s_w[threadIdx.x][i];
+    wsOut->part[threadIdx.x][blockIdx.x] = t;
   }
 }
 
@@ -733,7 +752,7 @@ extern "C" int libp_pcg_jacobi_csr_cg1_f64(int Nrows, const int* rowStarts, cons
     return arg_error("pcg_jacobi_csr_cg1", "null pointer");
   if (mode < 0 || mode > 3 || (parity & ~1)) return arg_error("pcg_jacobi_csr_cg1", "mode 0..3, parity 0 or 1");
   hipStream_t st = as_stream(stream);
-  const int nb = (Nrows + CSR_ROWS - 1) / CSR_ROWS < RMAXB ? (Nrows + CSR_ROWS - 1) / CSR_ROWS : RMAXB;
+  const int nb = csr_blocks(Nrows);
   ReduceWS* w = (ReduceWS*)ws;  // two workspaces, used by parity
   const int a = parity, b = parity ^ 1;
   if (mode == 3) {
@@ -744,8 +763,12 @@ extern "C" int libp_pcg_jacobi_csr_cg1_f64(int Nrows, const int* rowStarts, cons
   }
   const CG1Vec cur{p2[a], s2[a], r2[a], u2[a]}, nxt{p2[b], s2[b], r2[b], u2[b]};
   // mode 0 writes w[a], which iteration 0 (mode 1, parity a) reads
-  hipLaunchKernelGGL(coarse_cg1_csr_kernel, dim3(nb), dim3(CSR_THREADS), 0, st, Nrows, rowStarts, colIds, vals, mode,
-                     parity, tol * tol, nb, invDiag, x, cur, nxt, w2[a], w2[b], scalars, (const ReduceWS*)(w + a),
+  const int threads = csr_threads(Nrows);
+  const auto kernel = threads == 256   ? coarse_cg1_csr_kernel<256>
+                      : threads == 512 ? coarse_cg1_csr_kernel<512>
+                                       : coarse_cg1_csr_kernel<1024>;
+  hipLaunchKernelGGL(kernel, dim3(nb), dim3(threads), 0, st, Nrows, rowStarts, colIds, vals, mode, parity,
+                     tol * tol, nb, invDiag, x, cur, nxt, w2[a], w2[b], scalars, (const ReduceWS*)(w + a),
                      w + (mode == 0 ? a : b));
   return launch_status("pcg_jacobi_csr_cg1");
 }
@@ -755,7 +778,7 @@ extern "C" int libp_pcg_jacobi_csr_cg1_check_f64(int Nrows, int parity, double* 
   if (Nrows <= 0) return LIBP_OK;
   if (!scalars || !ws) return arg_error("pcg_jacobi_csr_cg1_check", "null pointer");
   if (parity & ~1) return arg_error("pcg_jacobi_csr_cg1_check", "parity 0 or 1");
-  const int nb = (Nrows + CSR_ROWS - 1) / CSR_ROWS < RMAXB ? (Nrows + CSR_ROWS - 1) / CSR_ROWS : RMAXB;
+  const int nb = csr_blocks(Nrows);
   // iteration (mode 1 or 2) of parity p wrote its partials to workspace p ^ 1
   hipLaunchKernelGGL(coarse_cg1_check_kernel, dim3(1), dim3(64), 0, as_stream(stream), nb, scalars,
                      (const ReduceWS*)ws + (parity ^ 1), hostMirror);
