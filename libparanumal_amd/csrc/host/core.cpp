@@ -2,7 +2,9 @@
 #include "core.hpp"
 
 #include <cctype>
+#include <deque>
 #include <iostream>
+#include <mutex>
 
 namespace libp {
 
@@ -196,6 +198,40 @@ settings_t ellipticDefaultSettings() {
   return s;
 }
 
+namespace {
+// Buffers waiting to be reused; any thread may return one.
+struct workspacePool {
+  static constexpr size_t MOST = 16;
+  std::mutex m;
+  std::deque<std::pair<size_t, void*>> waiting;
+  void* take(size_t bytes) {
+    std::lock_guard<std::mutex> lock(m);
+    for (auto it = waiting.rbegin(); it != waiting.rend(); ++it)
+      if (it->first == bytes) {
+        void* p = it->second;
+        waiting.erase(std::next(it).base());
+        return p;
+      }
+    return nullptr;
+  }
+  void give(void* p, size_t bytes) {
+    void* old = nullptr;
+    {
+      std::lock_guard<std::mutex> lock(m);
+      waiting.emplace_back(bytes, p);
+      if (waiting.size() > MOST) {
+        old = waiting.front().second;
+        waiting.pop_front();
+      }
+    }
+    if (old) (void)hipFree(old);
+  }
+  ~workspacePool() {
+    for (auto& w : waiting) (void)hipFree(w.second);
+  }
+};
+}  // namespace
+
 platform_t::platform_t(const settings_t& s) {
   int dev = 0;
   s.getSetting("DEVICE NUMBER", dev);
@@ -211,7 +247,7 @@ platform_t::platform_t(const settings_t& s) {
   LIBP_HIP(hipHostMalloc((void**)&pinned, 48 * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
   hipEvent_t ev = nullptr;
   LIBP_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-  struct State {
+  struct State : workspacePool {
     hipStream_t st = nullptr;
     double* pinned = nullptr;
     hipEvent_t ev = nullptr, pipe[2] = {nullptr, nullptr};
@@ -229,6 +265,7 @@ platform_t::platform_t(const settings_t& s) {
   stt->pinned = pinned;
   stt->ev = ev;
   state = stt;
+  pool_ = static_cast<workspacePool*>(stt.get());
   stream = st;
   h_scalars = pinned;
   ev_read = ev;
@@ -244,6 +281,20 @@ platform_t::platform_t(const settings_t& s) {
   o_scalars = deviceMemory<double>::alloc(64);
   LIBP_HIP(hipMemsetAsync(o_scalars.ptr(), 0, 64 * sizeof(double), stream));
   finish();
+}
+
+std::shared_ptr<void> platform_t::workspaceBytes(size_t bytes) const {
+  auto pool = std::static_pointer_cast<workspacePool>(std::shared_ptr<void>(state, pool_));
+  void* p = pool->take(bytes);
+  if (!p) LIBP_HIP(hipMalloc(&p, bytes));
+  // the buffer returns to the pool while the platform lives, and is freed after it
+  std::weak_ptr<workspacePool> home = pool;
+  return std::shared_ptr<void>(p, [home, bytes](void* q) {
+    if (auto h = home.lock())
+      h->give(q, bytes);
+    else
+      (void)hipFree(q);
+  });
 }
 
 const double* platform_t::readScalars(const double* dptr, int count) const {

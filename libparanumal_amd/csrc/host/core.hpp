@@ -100,6 +100,14 @@ class deviceMemory {
     m.n = count;
     return m;
   }
+  // Owning memory whose release is the caller's (platform_t::workspace).
+  static deviceMemory own(std::shared_ptr<void> base, size_t count) {
+    deviceMemory m;
+    m.p = static_cast<T*>(base.get());
+    m.n = count;
+    m.base = std::move(base);
+    return m;
+  }
   // Non-owning view of caller memory (C ABI entry points).
   static deviceMemory wrap(T* ptr, size_t count) {
     deviceMemory m;
@@ -178,6 +186,7 @@ class platform_t {
   int device = 0;
   hipStream_t stream = nullptr;
   std::shared_ptr<void> state;  // owns stream + buffers
+  void* pool_ = nullptr;        // the workspace pool inside state
   deviceMemory<char> o_reduceWS;
   deviceMemory<double> o_scalars;  // general-purpose device scalars
   double* h_scalars = nullptr;     // pinned mirror (16 doubles), mapped for the device
@@ -207,6 +216,16 @@ class platform_t {
     d.copyFrom(h.data(), h.size(), 0, stream);
     return d;
   }
+  // Device memory for work on this platform's stream, kept for the next caller of the same
+  // size when its last holder lets go of it: a solve's vectors (elliptic_t::Run makes about
+  // a dozen) cost ~0.15 ms each to allocate and free, 1.9 of the 10.2 ms of a whole p-MG
+  // call on 2.9M nodes. Reuse is ordered by the stream. At most 16 buffers wait (the
+  // oldest is freed), and all are freed with the platform.
+  template <typename T>
+  deviceMemory<T> workspace(size_t n) const {
+    return n == 0 ? deviceMemory<T>() : deviceMemory<T>::own(workspaceBytes(n * sizeof(T)), n);
+  }
+  std::shared_ptr<void> workspaceBytes(size_t bytes) const;
   void finish() const { LIBP_HIP(hipStreamSynchronize(stream)); }
   void* s() const { return (void*)stream; }
   // Reads device scalars [0,count) of ptr into the pinned buffer: a kernel

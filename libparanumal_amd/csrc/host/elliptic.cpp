@@ -390,8 +390,8 @@ ellipticRunResult_t elliptic_t::Run(int verboseOverride) {
   const int kind = dataKind();
   deviceMemory<dfloat> o_coeffs = dataCoefficients();
   const dlong NL = mesh.Nelements * mesh.Np;
-  deviceMemory<dfloat> o_rL = platform.malloc<dfloat>(NL), o_xL = platform.malloc<dfloat>(NL);
-  deviceMemory<dfloat> o_ubL = platform.malloc<dfloat>(NL), o_AubL = platform.malloc<dfloat>(NL);
+  deviceMemory<dfloat> o_rL = platform.workspace<dfloat>(NL), o_xL = platform.workspace<dfloat>(NL);
+  deviceMemory<dfloat> o_ubL = platform.workspace<dfloat>(NL), o_AubL = platform.workspace<dfloat>(NL);
   LIBP_CALL(libp_set_f64(NL, 0.0, o_xL.ptr(), platform.s()));
   // forcing (ellipticRhsHex3D.okl) and Dirichlet lift (ellipticRhsBCHex3D.okl: rhs -= A_L u_b)
   LIBP_CALL(libp_rhs_hex_f64(mesh.Nelements, mesh.Np, kind, o_coeffs.ptr(), mesh.o_x.ptr(), mesh.o_y.ptr(),
@@ -401,7 +401,7 @@ ellipticRunResult_t elliptic_t::Run(int verboseOverride) {
                                   o_ubL.ptr(), o_AubL.ptr(), platform.s()));
   LIBP_CALL(libp_axpy_f64(NL, -1.0, o_AubL.ptr(), 1.0, o_rL.ptr(), platform.s()));
 
-  deviceMemory<dfloat> o_r = platform.malloc<dfloat>(Ndofs + Nhalo), o_x = platform.malloc<dfloat>(Ndofs + Nhalo);
+  deviceMemory<dfloat> o_r = platform.workspace<dfloat>(Ndofs + Nhalo), o_x = platform.workspace<dfloat>(Ndofs + Nhalo);
   ogsMasked.Gather(o_r, o_rL, 1, ogs::Add, ogs::Trans);
   ogsMasked.Gather(o_x, o_xL, 1, ogs::Add, ogs::NoTrans);
 

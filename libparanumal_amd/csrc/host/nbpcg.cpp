@@ -17,13 +17,13 @@ const int NSC = 8;
 nbpcg::nbpcg(dlong _N, dlong _Nhalo, platform_t& _platform, settings_t& _settings, comm_t _comm)
     : linearSolverBase_t(_N, _Nhalo, _platform, _settings, _comm) {
   const dlong Nt = N + Nhalo;
-  o_p = platform.malloc<dfloat>(Nt);
-  o_s = platform.malloc<dfloat>(Nt);
-  o_S = platform.malloc<dfloat>(Nt);
-  o_z = platform.malloc<dfloat>(Nt);
-  o_Z = platform.malloc<dfloat>(Nt);
-  o_Ax = platform.malloc<dfloat>(Nt);
-  o_sc = platform.malloc<dfloat>(NSC);
+  o_p = platform.workspace<dfloat>(Nt);
+  o_s = platform.workspace<dfloat>(Nt);
+  o_S = platform.workspace<dfloat>(Nt);
+  o_z = platform.workspace<dfloat>(Nt);
+  o_Z = platform.workspace<dfloat>(Nt);
+  o_Ax = platform.workspace<dfloat>(Nt);
+  o_sc = platform.workspace<dfloat>(NSC);
   for (auto* v : {&o_p, &o_s, &o_S, &o_z, &o_Z, &o_Ax}) LIBP_CALL(libp_set_f64(Nt, 0.0, v->ptr(), platform.s()));
 }
 
@@ -67,10 +67,10 @@ nbfpcg::nbfpcg(dlong _N, dlong _Nhalo, platform_t& _platform, settings_t& _setti
     : linearSolverBase_t(_N, _Nhalo, _platform, _settings, _comm) {
   const dlong Nt = N + Nhalo;
   for (auto* v : {&o_u, &o_p, &o_w, &o_n, &o_m, &o_s, &o_z, &o_q, &o_Ax}) {
-    *v = platform.malloc<dfloat>(Nt);
+    *v = platform.workspace<dfloat>(Nt);
     LIBP_CALL(libp_set_f64(Nt, 0.0, v->ptr(), platform.s()));
   }
-  o_sc = platform.malloc<dfloat>(NSC);
+  o_sc = platform.workspace<dfloat>(NSC);
 }
 
 int nbfpcg::Solve(operator_t& A, operator_t& M, deviceMemory<dfloat>& o_x, deviceMemory<dfloat>& o_r,

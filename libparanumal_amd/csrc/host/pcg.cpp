@@ -14,12 +14,12 @@ pcg::pcg(dlong _N, dlong _Nhalo, platform_t& _platform, settings_t& _settings, c
   fuseJacobi = !settings.compareSetting("PCG JACOBI FUSED", "FALSE");
   if (settings.hasSetting("LINEAR SOLVER CHECK EVERY")) settings.getSetting("LINEAR SOLVER CHECK EVERY", checkEvery);
   const dlong Ntotal = N + Nhalo;
-  o_p = platform.malloc<dfloat>(Ntotal);
-  o_z = platform.malloc<dfloat>(Ntotal);
-  o_Ax = platform.malloc<dfloat>(Ntotal);
-  o_Ap = platform.malloc<dfloat>(Ntotal);
-  o_s = platform.malloc<dfloat>(LIBP_PCG_NSCALARS);
-  o_states = platform.malloc<dfloat>(32);
+  o_p = platform.workspace<dfloat>(Ntotal);
+  o_z = platform.workspace<dfloat>(Ntotal);
+  o_Ax = platform.workspace<dfloat>(Ntotal);
+  o_Ap = platform.workspace<dfloat>(Ntotal);
+  o_s = platform.workspace<dfloat>(LIBP_PCG_NSCALARS);
+  o_states = platform.workspace<dfloat>(32);
   // zero work vectors (linearSolverPCG.cpp:45-50 fills them with 0)
   LIBP_CALL(libp_set_f64(Ntotal, 0.0, o_p.ptr(), platform.s()));
   LIBP_CALL(libp_set_f64(Ntotal, 0.0, o_z.ptr(), platform.s()));
