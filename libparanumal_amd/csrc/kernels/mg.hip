@@ -1,122 +1,211 @@
 // p-multigrid intergrid transfers for hex elements (FP64 and FP32).
 //
-// One workgroup per element with an NqF x NqF thread tile; the three 1-D
-// contractions with P (NqF x NqC) run as successive sweeps through LDS, as in
-// okl/ellipticPreconCoarsenHex3D.okl:209-294 and
-// okl/ellipticPreconProlongateHex3D.okl:216-301. The reference uses NqF^3
-// threads, which exceeds the 1024-lane workgroup limit for N >= 10; the 2-D
-// tile looping over the third index covers every degree up to 15. NQC > 0
-// fixes the coarse size at compile time (the 7->3 and 3->1 steps of the
-// default schedule), so the sweeps unroll; NQC = 0 takes it at run time. The
-// arithmetic and its order are the same either way.
+// Each transfer is three 1-D contractions with P (NqF x NqC): k, j, i for the
+// restriction (okl/ellipticPreconCoarsenHex3D.okl:209-294), i, j, k for the
+// prolongation (okl/ellipticPreconProlongateHex3D.okl:216-301). A workgroup takes
+// NE elements. Their nodes are read and written flat (consecutive threads,
+// consecutive nodes), and in a contraction a thread holds one whole line: both
+// sizes are template arguments, so the line sits in registers, and the entries of
+// P, the same for every lane, come through scalar loads (a coarse size known only at
+// run time loads P entry by entry: 10->9 in FP32 took 45 us against 30).
+//
+// The form before took a NqF x NqF tile per element (the same arithmetic and order,
+// bit for bit), read P from LDS for every product, left lanes idle (49 of 64 at
+// NqF = 7) and had known sizes at 7->3 and 3->1 only. What bounds this one: HBM (12
+// bytes per fine node with the weights, FP32), and for the restriction the latency
+// of its index -> value loads. 8M fine nodes, microseconds, restriction / prolongation
+// before and now:
+//             2->1      3->1      4->2      6->4      7->3      9->6     12->9     15->11
+//   FP64    105/106     61/32     42/41     52/38     39/15     50/53     54/63     56/83
+//      now   31/22      30/17     30/20     35/24     32/17     43/24     44/30     45/38
+//   FP32     92/101     45/30     32/38     35/31     26/9.8    34/36     31/35     32/42
+//      now   24/17      21/12     23/14     26/16     23/10.5   27/15     24/19     24/20
 #include "kcommon.hpp"
 
 namespace libp_amd {
 
-template <int NqF, int NQC, typename T>
-__global__ void __launch_bounds__(NqF * NqF) mg_coarsen_kernel(const int NqC_, const int* __restrict__ elementList,
-                                                               const int* __restrict__ G2L, const T* __restrict__ P,
-                                                               const T* __restrict__ qf, const T* __restrict__ w,
-                                                               T* __restrict__ qc) {
-  constexpr int NpF = NqF * NqF * NqF;
-  // LDS: s_f is dead after the k sweep, so the j sweep writes into it (s_ccf).
-  // Sizes keep NqF=16 in FP64 within 64 KiB.
-  __shared__ T s_f[NqF][NqF][NqF];
-  __shared__ T s_cff[NqF - 1][NqF][NqF];
-  __shared__ T s_P[NqF][NqF - 1];
-  T(*s_ccf)[NqF][NqF] = s_f;
-  const int NqC = NQC > 0 ? NQC : NqC_;
-  const int e = blockIdx.x;
-  const int element = elementList ? elementList[e] : e;
-  const int t = threadIdx.x, i = t % NqF, j = t / NqF;
-  const int NpC = NqC * NqC * NqC;
+// Elements and threads per workgroup: about 1000 nodes, and threads for all the
+// fine lines of one direction where that is a multiple of a wavefront or close to it.
+// 7->3 at 1 element / 64 threads, 2 / 128 and 4 / 256 prolongs in 17.6, 16.7 and
+// 16.7 us (FP64); the tile form took 15.3 there, and 40 against 33 to restrict.
+template <int NqF>
+struct MgShape {
+  static constexpr int NE = NqF <= 3 ? 32 : NqF <= 5 ? 8 : NqF <= 7 ? 4 : NqF == 8 ? 2 : 1;
+  static constexpr int threads = (NqF >= 8 && NqF <= 11) || NqF == 4 ? 128 : 256;
+};
+
+template <int NqF, int NqC, typename T>
+__global__ void __launch_bounds__(MgShape<NqF>::threads)
+    mg_coarsen_kernel(const int Nelements, const int* __restrict__ elementList,
+                      const int* __restrict__ G2L, const T* __restrict__ P, const T* __restrict__ qf,
+                      const T* __restrict__ w, T* __restrict__ qc) {
+  constexpr int NE = MgShape<NqF>::NE, B = MgShape<NqF>::threads, FF = NqF * NqF, NpF = NqF * FF, NN = NE * NpF;
+  constexpr int UN = (NN + B - 1) / B, R = NqF | 1;  // rows of the last contraction, odd stride
+  __shared__ T s_f[NE * (NqF - 1) * (NqF - 1) * R > NN ? NE * (NqF - 1) * (NqF - 1) * R : NN];
+  __shared__ T s_c[NE * (NqF - 1) * FF];
+  const int t = threadIdx.x, e0 = blockIdx.x * NE, last = Nelements - 1 - e0;
+  const auto element = [&](const int es) {  // a group past the end repeats its last element
+    const int e = e0 + min(es, last);
+    return (size_t)(elementList ? elementList[e] : e);
+  };
   // index loads first, then unconditional value loads (masked nodes read entry 0 and take 0):
   // loads under (id >= 0) compile to branches that wait for each load in turn
-  int ids[NqF];
+  int ids[UN];
+  T q[UN], wv[UN];
 #pragma unroll
-  for (int k = 0; k < NqF; ++k) ids[k] = G2L[(size_t)element * NpF + k * NqF * NqF + t];
+  for (int u = 0; u < UN; ++u) {
+    const int n = min(t + u * B, NN - 1);
+    ids[u] = __builtin_nontemporal_load(G2L + element(n / NpF) * NpF + n % NpF);
+  }
 #pragma unroll
-  for (int k = 0; k < NqF; ++k) {
-    const int id = max(ids[k], 0);
+  for (int u = 0; u < UN; ++u) {
+    const int id = max(ids[u], 0);
+    q[u] = qf[id];
     // w: the inverse-multiplicity weight of the fine residual (ellipticPreconMultiGridLevel.cpp:51),
     // applied here instead of in a separate pass (the same single rounding)
-    const T qv = qf[id];
-    const T wv = w ? w[id] : T(1);
-    s_f[k][j][i] = (ids[k] >= 0) ? (w ? T(1) * wv * qv : qv) : T(0);
+    if (w) wv[u] = w[id];
   }
-  if (t < NqF * NqC) s_P[t / NqC][t % NqC] = P[t];
+#pragma unroll
+  for (int u = 0; u < UN; ++u)
+    if ((u + 1) * B <= NN || t + u * B < NN)
+      s_f[t + u * B] = (ids[u] >= 0) ? (w ? T(1) * wv[u] * q[u] : q[u]) : T(0);
   __syncthreads();
-  for (int k = 0; k < NqC; ++k) {
-    T res = 0;
-    for (int m = 0; m < NqF; ++m) res += s_P[m][k] * s_f[m][j][i];
-    s_cff[k][j][i] = res;
+  // k: lines (e, j, i) of s_f -> s_c[e][c][j][i]
+  for (int p = t; p < NE * FF; p += B) {
+    const int e = p / FF, ji = p % FF;
+    T x[NqF];
+#pragma unroll
+    for (int m = 0; m < NqF; ++m) x[m] = s_f[e * NpF + m * FF + ji];
+    for (int c = 0; c < NqC; ++c) {
+      T res = 0;
+#pragma unroll
+      for (int m = 0; m < NqF; ++m) res += P[m * NqC + c] * x[m];
+      s_c[(e * NqC + c) * FF + ji] = res;
+    }
   }
   __syncthreads();
-  if (j < NqC)
-    for (int k = 0; k < NqC; ++k) {
+  // j: lines (e, k, i) of s_c -> s_f[e][k][c][i], rows of R
+  for (int p = t; p < NE * NqC * NqF; p += B) {
+    const int ek = p / NqF, i = p % NqF;
+    T x[NqF];
+#pragma unroll
+    for (int m = 0; m < NqF; ++m) x[m] = s_c[ek * FF + m * NqF + i];
+    for (int c = 0; c < NqC; ++c) {
       T res = 0;
-      for (int m = 0; m < NqF; ++m) res += s_P[m][j] * s_cff[k][m][i];
-      s_ccf[k][j][i] = res;
+#pragma unroll
+      for (int m = 0; m < NqF; ++m) res += P[m * NqC + c] * x[m];
+      s_f[(ek * NqC + c) * R + i] = res;
     }
+  }
   __syncthreads();
-  if (i < NqC && j < NqC) {
-    for (int k = 0; k < NqC; ++k) {
+  // i: lines (e, k, j) of s_f -> s_c, flat coarse nodes
+  for (int p = t; p < NE * NqC * NqC; p += B) {
+    T x[NqF];
+#pragma unroll
+    for (int m = 0; m < NqF; ++m) x[m] = s_f[p * R + m];
+    for (int c = 0; c < NqC; ++c) {
       T res = 0;
-      for (int m = 0; m < NqF; ++m) res += s_P[m][i] * s_ccf[k][j][m];
-      qc[(size_t)element * NpC + i + j * NqC + k * NqC * NqC] = res;
+#pragma unroll
+      for (int m = 0; m < NqF; ++m) res += P[m * NqC + c] * x[m];
+      s_c[p * NqC + c] = res;
     }
+  }
+  __syncthreads();
+  const int NpC = NqC * NqC * NqC;
+  for (int n = t; n < NE * NpC; n += B) {
+    const int e = n / NpC;
+    qc[element(e) * NpC + (n - e * NpC)] = s_c[n];
   }
 }
 
-template <int NqF, int NQC, typename T>
-__global__ void __launch_bounds__(NqF * NqF) mg_prolong_kernel(const int NqC_, const int* __restrict__ elementList,
-                                                               const int* __restrict__ G2LC, const T* __restrict__ P,
-                                                               const T* __restrict__ qcIn, T* __restrict__ qN) {
-  constexpr int NpF = NqF * NqF * NqF;
-  // LDS: s_ccc is dead after the i sweep, so the j sweep writes into it (s_cff).
-  __shared__ T s_A[NqF - 1][NqF][NqF];
-  __shared__ T s_ccf[NqF - 1][NqF - 1][NqF];
-  __shared__ T s_P[NqF][NqF - 1];
-  T(*s_ccc)[NqF][NqF] = s_A;
-  T(*s_cff)[NqF][NqF] = s_A;
-  const int NqC = NQC > 0 ? NQC : NqC_;
-  const int e = blockIdx.x;
-  const int element = elementList ? elementList[e] : e;
-  const int t = threadIdx.x, i = t % NqF, j = t / NqF;
-  const int NpC = NqC * NqC * NqC;
-  if (i < NqC && j < NqC) {
-    // index loads first, then unconditional value loads (a masked node reads entry 0 and
-    // takes 0); NqC < NqF, and k < NqC is the same for every lane
-    int ids[NqF - 1];
+template <int NqF, int NqC, typename T>
+__global__ void __launch_bounds__(MgShape<NqF>::threads)
+    mg_prolong_kernel(const int Nelements, const int* __restrict__ elementList,
+                      const int* __restrict__ G2LC, const T* __restrict__ P, const T* __restrict__ qcIn,
+                      T* __restrict__ qN) {
+  constexpr int NE = MgShape<NqF>::NE, B = MgShape<NqF>::threads, FF = NqF * NqF, NpF = NqF * FF, C = NqF - 1;
+  constexpr int UN = (NE * C * C * C + B - 1) / B;
+  __shared__ T s_c[NE * C * NqF * NqF];  // coarse nodes, then [e][k][j fine][i fine]
+  __shared__ T s_m[NE * C * C * NqF];    // [e][k][j][i fine]
+  const int t = threadIdx.x, e0 = blockIdx.x * NE, last = Nelements - 1 - e0;
+  const auto element = [&](const int es) {
+    const int e = e0 + min(es, last);
+    return (size_t)(elementList ? elementList[e] : e);
+  };
+  const int NpC = NqC * NqC * NqC, NC = NE * NpC;
+  // index loads first, then unconditional value loads; u * B < NC is the same for every lane
+  int ids[UN];
 #pragma unroll
-    for (int k = 0; k < NqF - 1; ++k)
-      if (k < NqC) ids[k] = G2LC[(size_t)element * NpC + i + j * NqC + k * NqC * NqC];
-#pragma unroll
-    for (int k = 0; k < NqF - 1; ++k)
-      if (k < NqC) {
-        const T qv = qcIn[max(ids[k], 0)];
-        s_ccc[k][j][i] = (ids[k] >= 0) ? qv : T(0);
-      }
-  }
-  if (t < NqF * NqC) s_P[t / NqC][t % NqC] = P[t];
-  __syncthreads();
-  if (j < NqC)
-    for (int k = 0; k < NqC; ++k) {
-      T res = 0;
-      for (int m = 0; m < NqC; ++m) res += s_P[i][m] * s_ccc[k][j][m];
-      s_ccf[k][j][i] = res;
+  for (int u = 0; u < UN; ++u)
+    if (u * B < NC) {
+      const int n = min(t + u * B, NC - 1), e = n / NpC;
+      ids[u] = __builtin_nontemporal_load(G2LC + element(e) * NpC + (n - e * NpC));
     }
+  T q[UN];
+#pragma unroll
+  for (int u = 0; u < UN; ++u)
+    if (u * B < NC) q[u] = qcIn[max(ids[u], 0)];
+#pragma unroll
+  for (int u = 0; u < UN; ++u)
+    if (t + u * B < NC) s_c[t + u * B] = (ids[u] >= 0) ? q[u] : T(0);
   __syncthreads();
-  for (int k = 0; k < NqC; ++k) {
-    T res = 0;
-    for (int m = 0; m < NqC; ++m) res += s_P[j][m] * s_ccf[k][m][i];
-    s_cff[k][j][i] = res;
+  // i: lines (e, k, j) -> s_m
+  for (int p = t; p < NE * NqC * NqC; p += B) {
+    T o[NqF];
+#pragma unroll
+    for (int f = 0; f < NqF; ++f) o[f] = 0;
+    for (int m = 0; m < NqC; ++m) {
+      const T x = s_c[p * NqC + m];
+#pragma unroll
+      for (int f = 0; f < NqF; ++f) o[f] += P[f * NqC + m] * x;
+    }
+#pragma unroll
+    for (int f = 0; f < NqF; ++f) s_m[p * NqF + f] = o[f];
   }
   __syncthreads();
-  for (int k = 0; k < NqF; ++k) {
-    T res = 0;
-    for (int m = 0; m < NqC; ++m) res += s_P[k][m] * s_cff[m][j][i];
-    qN[(size_t)element * NpF + i + j * NqF + k * NqF * NqF] = res;
+  // j: lines (e, k, i) -> s_c
+  for (int p = t; p < NE * NqC * NqF; p += B) {
+    const int ek = p / NqF, i = p % NqF;
+    T o[NqF];
+#pragma unroll
+    for (int f = 0; f < NqF; ++f) o[f] = 0;
+    for (int m = 0; m < NqC; ++m) {
+      const T x = s_m[(ek * NqC + m) * NqF + i];
+#pragma unroll
+      for (int f = 0; f < NqF; ++f) o[f] += P[f * NqC + m] * x;
+    }
+#pragma unroll
+    for (int f = 0; f < NqF; ++f) s_c[ek * FF + f * NqF + i] = o[f];
+  }
+  __syncthreads();
+  // k: lines (e, j, i) -> the E-vector; at each f a run of consecutive nodes
+  for (int p = t; p < NE * FF; p += B) {
+    const int e = p / FF, ji = p % FF;
+    T o[NqF];
+#pragma unroll
+    for (int f = 0; f < NqF; ++f) o[f] = 0;
+    for (int m = 0; m < NqC; ++m) {
+      const T x = s_c[(e * NqC + m) * FF + ji];
+#pragma unroll
+      for (int f = 0; f < NqF; ++f) o[f] += P[f * NqC + m] * x;
+    }
+    T* out = qN + element(e) * NpF + ji;
+#pragma unroll
+    for (int f = 0; f < NqF; ++f) out[f * FF] = o[f];
+  }
+}
+
+// the kernel of coarse size nqc, NqC <= nqc < NqF
+template <int NqF, int NqC, typename T, bool COARSEN>
+static void launch_transfer(int nqc, int Nelements, const int* elist, const int* g2l, const T* P, const T* in,
+                            const T* w, T* out, hipStream_t st) {
+  if constexpr (NqC < NqF) {
+    if (nqc != NqC) return launch_transfer<NqF, NqC + 1, T, COARSEN>(nqc, Nelements, elist, g2l, P, in, w, out, st);
+    const dim3 grid((Nelements + MgShape<NqF>::NE - 1) / MgShape<NqF>::NE), block(MgShape<NqF>::threads);
+    if constexpr (COARSEN)
+      hipLaunchKernelGGL((mg_coarsen_kernel<NqF, NqC, T>), grid, block, 0, st, Nelements, elist, g2l, P, in, w, out);
+    else
+      hipLaunchKernelGGL((mg_prolong_kernel<NqF, NqC, T>), grid, block, 0, st, Nelements, elist, g2l, P, in, out);
   }
 }
 
@@ -127,34 +216,12 @@ static int transfer(int Nf, int Nc, int Nelements, const int* elist, const int* 
   if (Nc < 1 || Nc >= Nf || Nf > 15) return arg_error("mg_transfer", "need 1 <= Nc < Nf <= 15");
   if (!g2l || !P || !in || !out) return arg_error("mg_transfer", "null pointer");
   hipStream_t st = as_stream(stream);
-  const int NqC = Nc + 1;
-  // the default schedule's steps with the coarse size fixed at compile time
-  if (Nf == 7 && Nc == 3) {
-    if (COARSEN)
-      hipLaunchKernelGGL((mg_coarsen_kernel<8, 4, T>), dim3(Nelements), dim3(64), 0, st, NqC, elist, g2l, P, in, w,
-                         out);
-    else
-      hipLaunchKernelGGL((mg_prolong_kernel<8, 4, T>), dim3(Nelements), dim3(64), 0, st, NqC, elist, g2l, P, in, out);
-    return launch_status(COARSEN ? "mg_coarsen" : "mg_prolong");
-  }
-  if (Nf == 3 && Nc == 1) {
-    if (COARSEN)
-      hipLaunchKernelGGL((mg_coarsen_kernel<4, 2, T>), dim3(Nelements), dim3(16), 0, st, NqC, elist, g2l, P, in, w,
-                         out);
-    else
-      hipLaunchKernelGGL((mg_prolong_kernel<4, 2, T>), dim3(Nelements), dim3(16), 0, st, NqC, elist, g2l, P, in, out);
-    return launch_status(COARSEN ? "mg_coarsen" : "mg_prolong");
-  }
-  switch (Nf + 1) {
-#define LIBP_MG_CASE(NQ)                                                                                            \
-  case NQ:                                                                                                          \
-    if (COARSEN)                                                                                                    \
-      hipLaunchKernelGGL((mg_coarsen_kernel<NQ, 0, T>), dim3(Nelements), dim3(NQ * NQ), 0, st, NqC, elist, g2l, P, \
-                         in, w, out);                                                                               \
-    else                                                                                                            \
-      hipLaunchKernelGGL((mg_prolong_kernel<NQ, 0, T>), dim3(Nelements), dim3(NQ * NQ), 0, st, NqC, elist, g2l, P,  \
-                         in, out);                                                                                  \
+  switch (Nf) {
+#define LIBP_MG_CASE(NF)                                                                     \
+  case NF:                                                                                   \
+    launch_transfer<NF + 1, 2, T, COARSEN>(Nc + 1, Nelements, elist, g2l, P, in, w, out, st); \
     break;
+    LIBP_MG_CASE(2)
     LIBP_MG_CASE(3)
     LIBP_MG_CASE(4)
     LIBP_MG_CASE(5)
@@ -168,7 +235,6 @@ static int transfer(int Nf, int Nc, int Nelements, const int* elist, const int* 
     LIBP_MG_CASE(13)
     LIBP_MG_CASE(14)
     LIBP_MG_CASE(15)
-    LIBP_MG_CASE(16)
 #undef LIBP_MG_CASE
     default:
       return arg_error("mg_transfer", "unsupported fine degree");
