@@ -501,7 +501,8 @@ int libp_mlp_linear_bwd_data(int M, int K, int Nout, const unsigned short* dY, l
                              void* stream);
 /* Weight gradients: dWt[Nout x K] = dY^T X (FP32, [Nout][K] dense) and
  * db[Nout] = column sums of dY (FP32, or NULL). Split-K over M with FP32
- * partials summed in a fixed order; ws holds libp_mlp_ws_bytes(M, K, Nout). */
+ * partials summed in a fixed order; ws holds libp_mlp_ws_bytes(M, K, Nout), which
+ * grows with each of its arguments: the largest call's workspace serves the others. */
 int libp_mlp_linear_bwd_weight(int M, int K, int Nout, const unsigned short* dY, long lddy, const unsigned short* X,
                                long ldx, float* dWt, float* db, void* ws, void* stream);
 long libp_mlp_ws_bytes(int M, int K, int Nout);

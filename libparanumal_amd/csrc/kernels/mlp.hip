@@ -649,9 +649,13 @@ extern "C" int libp_mlp_linear_bwd_data(int M, int K, int Nout, const unsigned s
 }
 
 extern "C" long libp_mlp_ws_bytes(int M, int K, int Nout) {
-  int S, kc;
-  weight_splits(M, K, Nout, S, kc);
-  return (long)S * Nout * K * 4 + (long)colsum_chunks(M) * Nout * 4 + 256;
+  // The splits of weight_splits fall as the tiles grow, so S * Nout * K does not grow with every
+  // size; what is asked for does, and a workspace of the largest call serves the smaller ones:
+  // S <= one per 256 rows and 64, and S * tiles < 512 + tiles (34 MB of splits beside the result).
+  const long rows = std::min(64L, (M + 255L) / 256), entries = (long)Nout * K;
+  const long tiles = ((K + GBN - 1L) / GBN) * ((Nout + GBM - 1L) / GBM);
+  const long splits = std::min(std::max(rows, 1L) * entries, (511 + tiles) * GBM * GBN);
+  return splits * 4 + (long)colsum_chunks(M) * Nout * 4 + 256;
 }
 
 extern "C" int libp_mlp_linear_bwd_weight(int M, int K, int Nout, const unsigned short* dY, long lddy,

@@ -56,10 +56,13 @@ def test_mlp_products_at_tile_edges(M, K, N):
         assert ((dX.double() - want).abs() <= bound + 2.0**-8 * want.abs()).all()
 
     dW, db = torch.full((N, K), nan, device="cuda"), torch.full((N,), nan, device="cuda")
-    ws = torch.full((L.libp_mlp_ws_bytes(M, K, N) // 4,), nan, device="cuda")
+    n_ws = L.libp_mlp_ws_bytes(M, K, N) // 4
+    ws = torch.full((n_ws + 4096,), nan, device="cuda")
+    ws[n_ws:] = 3.0  # past the workspace: stays
     lp.check(L.libp_mlp_linear_bwd_weight(M, K, N, dY.data_ptr(), N, X.data_ptr(), K, dW.data_ptr(), db.data_ptr(),
                                           ws.data_ptr(), st))
     torch.cuda.synchronize()
+    assert (ws[n_ws:] == 3.0).all()
     ref, bound = product(dY.T, X)
     assert ((dW.double() - ref).abs() <= bound).all()
     mag = dY.double().abs().sum(0)
