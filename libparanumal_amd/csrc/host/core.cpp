@@ -2,9 +2,7 @@
 #include "core.hpp"
 
 #include <cctype>
-#include <deque>
 #include <iostream>
-#include <mutex>
 
 namespace libp {
 
@@ -198,39 +196,21 @@ settings_t ellipticDefaultSettings() {
   return s;
 }
 
-namespace {
-// Buffers waiting to be reused; any thread may return one.
-struct workspacePool {
-  static constexpr size_t MOST = 16;
-  std::mutex m;
-  std::deque<std::pair<size_t, void*>> waiting;
-  void* take(size_t bytes) {
-    std::lock_guard<std::mutex> lock(m);
-    for (auto it = waiting.rbegin(); it != waiting.rend(); ++it)
-      if (it->first == bytes) {
-        void* p = it->second;
-        waiting.erase(std::next(it).base());
-        return p;
-      }
+static void freeDevice(void* p) { (void)hipFree(p); }
+
+void* deviceAlloc(size_t bytes) {
+  hipError_t e = hipSuccess;
+  void* p = workspacePool::allocate([&]() -> void* {
+    void* q = nullptr;
+    e = hipMalloc(&q, bytes);
+    if (e == hipSuccess) return q;
+    (void)hipGetLastError();  // handled here: not for the next launch to report
+    LIBP_ABORT("hipMalloc of " << bytes << " bytes failed: " << hipGetErrorString(e), e != hipErrorOutOfMemory);
     return nullptr;
-  }
-  void give(void* p, size_t bytes) {
-    void* old = nullptr;
-    {
-      std::lock_guard<std::mutex> lock(m);
-      waiting.emplace_back(bytes, p);
-      if (waiting.size() > MOST) {
-        old = waiting.front().second;
-        waiting.pop_front();
-      }
-    }
-    if (old) (void)hipFree(old);
-  }
-  ~workspacePool() {
-    for (auto& w : waiting) (void)hipFree(w.second);
-  }
-};
-}  // namespace
+  });
+  LIBP_ABORT("hipMalloc of " << bytes << " bytes failed: " << hipGetErrorString(e), !p);
+  return p;
+}
 
 platform_t::platform_t(const settings_t& s) {
   int dev = 0;
@@ -248,6 +228,7 @@ platform_t::platform_t(const settings_t& s) {
   hipEvent_t ev = nullptr;
   LIBP_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   struct State : workspacePool {
+    State() : workspacePool(freeDevice) {}
     hipStream_t st = nullptr;
     double* pinned = nullptr;
     hipEvent_t ev = nullptr, pipe[2] = {nullptr, nullptr};
@@ -286,7 +267,7 @@ platform_t::platform_t(const settings_t& s) {
 std::shared_ptr<void> platform_t::workspaceBytes(size_t bytes) const {
   auto pool = std::static_pointer_cast<workspacePool>(std::shared_ptr<void>(state, pool_));
   void* p = pool->take(bytes);
-  if (!p) LIBP_HIP(hipMalloc(&p, bytes));
+  if (!p) p = deviceAlloc(bytes);
   // the buffer returns to the pool while the platform lives, and is freed after it
   std::weak_ptr<workspacePool> home = pool;
   return std::shared_ptr<void>(p, [home, bytes](void* q) {

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "libp_amd.h"
+#include "workspace_pool.hpp"
 
 namespace libp {
 
@@ -56,6 +57,10 @@ class exception : public std::runtime_error {
     LIBP_ABORT(#expr << " failed: " << hipGetErrorString(_e), _e != hipSuccess);     \
   } while (0)
 
+// hipMalloc. Without memory for it, the buffers that wait in the platforms' pools are
+// freed and it is tried once more; then it throws.
+void* deviceAlloc(size_t bytes);
+
 /* Host array with shared (shallow-copy) ownership, like memory<T>
  * (include/memory.hpp:34-268). */
 template <typename T>
@@ -93,8 +98,7 @@ class deviceMemory {
   static deviceMemory alloc(size_t count) {
     deviceMemory m;
     if (count == 0) return m;
-    void* raw = nullptr;
-    LIBP_HIP(hipMalloc(&raw, count * sizeof(T)));
+    void* raw = deviceAlloc(count * sizeof(T));
     m.base = std::shared_ptr<void>(raw, [](void* q) { (void)hipFree(q); });
     m.p = static_cast<T*>(raw);
     m.n = count;
@@ -219,8 +223,9 @@ class platform_t {
   // Device memory for work on this platform's stream, kept for the next caller of the same
   // size when its last holder lets go of it: a solve's vectors (elliptic_t::Run makes about
   // a dozen) cost ~0.15 ms each to allocate and free, 1.9 of the 10.2 ms of a whole p-MG
-  // call on 2.9M nodes. Reuse is ordered by the stream. At most 16 buffers wait (the
-  // oldest is freed), and all are freed with the platform.
+  // call on 2.9M nodes. Reuse is ordered by the stream. At most 16 buffers and 512 MiB
+  // wait (the oldest are freed); all are freed with the platform, or when an allocation
+  // finds no memory.
   template <typename T>
   deviceMemory<T> workspace(size_t n) const {
     return n == 0 ? deviceMemory<T>() : deviceMemory<T>::own(workspaceBytes(n * sizeof(T)), n);
