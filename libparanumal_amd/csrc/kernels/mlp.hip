@@ -14,16 +14,21 @@
 // K tile, two workgroups per CU (the layers have 512 to 1024 tiles).
 // What bounds it: the LDS reads of a K tile take as long as its MFMAs, and with
 // two workgroups per CU little covers a tile's first loads and its epilogue.
-// 32,768 rows, microseconds before -> now: forward 896->256 37 -> 26 (0.58
-// PFLOP/s), 256->256 22 -> 14, 256->512 26 -> 25; data gradient 512->256 42 -> 22,
-// 256->256 33 -> 16; weight gradient 256x896 92 -> 34, 256x256 75 -> 15,
-// 512x256 78 -> 21; the column and split sums of the three 275 -> 40. Operands reach LDS as [row][k] (row stride 40 elements) whatever
-// their layout in HBM: a K-contiguous operand is copied with 16-byte loads and
+//
+// Operands reach LDS as [row][k] (row stride BK + 8 entries) whatever their
+// layout in HBM: a K-contiguous operand is copied with 16-byte loads and
 // stores; of a row-contiguous one (the transposed operands of the backward
 // products) each thread loads a 4 x 4 patch, four 8-byte loads, transposes it
-// with byte permutes and stores four 8-byte pieces. (With 16-byte loads and
-// sixteen 2-byte LDS stores per thread the LDS writes bound the kernel: dW of
-// 32,768 x 896 x 256 took 92 us, and 32,768 x 256 x 256 took 75.)
+// with byte permutes and stores four 8-byte pieces.
+//
+// Whole calls, ten in a replayed graph, 32,768 rows, microseconds; before: BK = 32,
+// four workgroups per CU, transposed operands stored to LDS two bytes at a time,
+// each chunk's load and each result's store under a branch of its own:
+//   layer        896->256    256->256    256->512   | 256->125    256->343    1000->1001
+//   forward       37 -> 27    22 -> 15    27 -> 25  |  20 -> 17    26 -> 25   153 -> 124
+//   data          96 -> 43    44 -> 16    61 -> 22  |  38 -> 35    59 -> 49   363 -> 284
+//   weight       235 -> 42   179 -> 27   182 -> 35  | 218 -> 41   224 -> 58   662 -> 246
+// (left: whole vectors everywhere, gemm_vectors; right: a width that is none).
 #include <algorithm>
 #include <cmath>
 
@@ -47,7 +52,7 @@ __device__ inline u16 f2bf(float f) {
 }
 __device__ inline float bf2f(u16 h) { return __builtin_bit_cast(float, (unsigned)h << 16); }
 
-constexpr int GBM = 128, GBN = 128, GBK = 64, GLD = GBK + 8;
+constexpr int GBM = 128, GBN = 128, GBK = 64;
 constexpr int GTHREADS = 256;
 
 enum { EPI_F32_BIAS = 0, EPI_BF16_BIAS_RELU = 1, EPI_BF16_MASK = 2, EPI_F32_PARTIAL = 3 };
@@ -66,80 +71,6 @@ struct GemmArgs {
   int kChunk;           // K range of one split (multiple of GBK)
   const float* rowScale = nullptr;  // EPI_F32_BIAS: C[m][n] = rowScale[m] * (A B + bias)[m][n] when set
 };
-
-// One operand tile (rows x GBK) in registers: GCH 16-byte chunks per thread.
-constexpr int GCH = GBM * GBK * 2 / 16 / GTHREADS;
-struct TileRegs {
-  u32x4 v[GCH];
-};
-
-// A tile inside the matrix (and aligned: vec) takes loads that no branch guards,
-// so that they are all in flight together; the others take them entry by entry.
-template <bool T>
-__device__ inline void load_tile(TileRegs& R, const u16* __restrict__ X, long ld, int row0, int nrows, int k0, int kEnd,
-                                 bool vec) {
-  const int t = threadIdx.x;
-  const bool whole = vec && row0 + GBM <= nrows && k0 + GBK <= kEnd;  // the same for every thread
-  if (T) {  // patch i: rows k0 + 32 i + 4 (t & 7) + r, r = 0..3; columns row0 + 4 (t >> 3) ..
-    const int gk0 = k0 + 4 * (t & 7), gr = row0 + 4 * (t >> 3);
-    if (whole) {
-#pragma unroll
-      for (int ir = 0; ir < 2 * GCH; ++ir) {
-        const u32x2 w = *reinterpret_cast<const u32x2*>(X + (long)(gk0 + 32 * (ir >> 2) + (ir & 3)) * ld + gr);
-        R.v[ir >> 1][2 * (ir & 1)] = w.x;
-        R.v[ir >> 1][2 * (ir & 1) + 1] = w.y;
-      }
-      return;
-    }
-#pragma unroll
-    for (int ir = 0; ir < 2 * GCH; ++ir) {
-      const int gk = gk0 + 32 * (ir >> 2) + (ir & 3);
-      u16 e[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) e[j] = (gk < kEnd && gr + j < nrows) ? X[(long)gk * ld + gr + j] : (u16)0;
-      R.v[ir >> 1][2 * (ir & 1)] = (unsigned)e[0] | ((unsigned)e[1] << 16);
-      R.v[ir >> 1][2 * (ir & 1) + 1] = (unsigned)e[2] | ((unsigned)e[3] << 16);
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < GCH; ++i) {
-    const int c = t + GTHREADS * i;
-    const int gr = row0 + c / (GBK / 8), gk = k0 + (c % (GBK / 8)) * 8;
-    if (whole) {
-      R.v[i] = *reinterpret_cast<const u32x4*>(X + (long)gr * ld + gk);
-      continue;
-    }
-    u16 tmp[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) tmp[e] = (gr < nrows && gk + e < kEnd) ? X[(long)gr * ld + gk + e] : (u16)0;
-    R.v[i] = u32x4{(unsigned)tmp[0] | ((unsigned)tmp[1] << 16), (unsigned)tmp[2] | ((unsigned)tmp[3] << 16),
-                   (unsigned)tmp[4] | ((unsigned)tmp[5] << 16), (unsigned)tmp[6] | ((unsigned)tmp[7] << 16)};
-  }
-}
-
-template <bool T>
-__device__ inline void store_tile(const TileRegs& R, u16* __restrict__ s) {
-  const int t = threadIdx.x;
-  if (T) {  // column j of the patch: k entries of four rows, low and high halves picked by byte
-#pragma unroll
-    for (int ij = 0; ij < 2 * GCH; ++ij) {
-      const int i = ij >> 2, j = ij & 3, d = j >> 1;
-      u16* o = s + 4 * (t >> 3) * GLD + 32 * i + 4 * (t & 7);
-      const unsigned pick = (j & 1) ? 0x07060302u : 0x05040100u;
-      *reinterpret_cast<u32x2*>(o + j * GLD) = u32x2{
-          __builtin_amdgcn_perm(R.v[2 * i][2 + d], R.v[2 * i][d], pick),
-          __builtin_amdgcn_perm(R.v[2 * i + 1][2 + d], R.v[2 * i + 1][d], pick)};
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < GCH; ++i) {
-    const int c = t + GTHREADS * i;
-    const int row = c / (GBK / 8), kc = (c % (GBK / 8)) * 8;
-    *reinterpret_cast<u32x4*>(s + row * GLD + kc) = R.v[i];
-  }
-}
 
 // Workgroups are dispatched round-robin over the eight XCDs, each with its
 // own L2. When the M tiles come in multiples of eight, the tiles are renamed
@@ -165,118 +96,26 @@ __device__ inline void gemm_tile(int& mt, int& nt, int& split) {
   }
 }
 
-template <bool TA, bool TB, int EPI>
-__global__ void __launch_bounds__(GTHREADS, 2) gemm_bf16_kernel(const GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) u16 sA[2][GBM * GLD];
-  __shared__ __attribute__((aligned(16))) u16 sB[2][GBN * GLD];
-  const int t = threadIdx.x, w = t >> 6, l = t & 63;
-  const int wm = w >> 1, wn = w & 1;
-  int mt, nt, split;
-  gemm_tile(mt, nt, split);
-  const int m0 = mt * GBM, n0 = nt * GBN;
-  const int kBeg = split * g.kChunk;
-  const int kEnd = min(g.K, kBeg + g.kChunk);
-  const bool vecA = (g.lda % 8) == 0 && ((uintptr_t)g.A & 15) == 0;
-  const bool vecB = (g.ldb % 8) == 0 && ((uintptr_t)g.B & 15) == 0;
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  const int nT = (kEnd > kBeg) ? (kEnd - kBeg + GBK - 1) / GBK : 0;
-  TileRegs ra, rb;
-  if (nT > 0) {
-    load_tile<TA>(ra, g.A, g.lda, m0, g.M, kBeg, kEnd, vecA);
-    load_tile<TB>(rb, g.B, g.ldb, n0, g.N, kBeg, kEnd, vecB);
-    store_tile<TA>(ra, sA[0]);
-    store_tile<TB>(rb, sB[0]);
-  }
-  __syncthreads();
-  const int lr = l & 31, lk = 8 * (l >> 5);
-  for (int it = 0; it < nT; ++it) {
-    const int buf = it & 1;
-    if (it + 1 < nT) {
-      const int k0 = kBeg + (it + 1) * GBK;
-      load_tile<TA>(ra, g.A, g.lda, m0, g.M, k0, kEnd, vecA);
-      load_tile<TB>(rb, g.B, g.ldb, n0, g.N, k0, kEnd, vecB);
-    }
-    const u16* a_s = sA[buf];
-    const u16* b_s = sB[buf];
-#pragma unroll
-    for (int ks = 0; ks < GBK; ks += 16) {
-      bf16x8 a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        a[i] = *reinterpret_cast<const bf16x8*>(a_s + (wm * 64 + i * 32 + lr) * GLD + ks + lk);
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        b[j] = *reinterpret_cast<const bf16x8*>(b_s + (wn * 64 + j * 32 + lr) * GLD + ks + lk);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-    if (it + 1 < nT) {
-      store_tile<TA>(ra, sA[buf ^ 1]);
-      store_tile<TB>(rb, sB[buf ^ 1]);
-    }
-    __syncthreads();
-  }
-
-  // epilogue
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = n0 + wn * 64 + j * 32 + lr;
-      if (col >= g.N) continue;
-      const float bcol = (g.bias && (EPI == EPI_F32_BIAS || EPI == EPI_BF16_BIAS_RELU)) ? g.bias[col] : 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
-        if (row >= g.M) continue;
-        const float v = acc[i][j][r];
-        if (EPI == EPI_F32_BIAS) {
-          const float o = v + bcol;
-          reinterpret_cast<float*>(g.C)[(long)row * g.ldc + col] = g.rowScale ? g.rowScale[row] * o : o;
-        } else if (EPI == EPI_BF16_BIAS_RELU) {
-          reinterpret_cast<u16*>(g.C)[(long)row * g.ldc + col] = f2bf(fmaxf(v + bcol, 0.f));
-        } else if (EPI == EPI_BF16_MASK) {
-          const bool keep = !g.mask || bf2f(g.mask[(long)row * g.ldm + col]) > 0.f;
-          reinterpret_cast<u16*>(g.C)[(long)row * g.ldc + col] = f2bf(keep ? v : 0.f);
-        } else {
-          reinterpret_cast<float*>(g.C)[(long)split * g.M * g.ldc + (long)row * g.ldc + col] = v;
-        }
-      }
-    }
-}
-
-// The same product where every access can be a whole vector (gemm_vectors below
-// says when): no load or store sits under a branch, so the loads of the next K
-// tile are all in flight during a tile's MFMAs. (Guarded per chunk, as in
-// gemm_bf16_kernel, each load was its own branch and each of the 64 two-byte
-// result stores waited for the one before it.) Rows past the end of A or B
-// repeat the last one (their results are not stored); K entries past the end of
-// a transposed operand are zeroed on the way to LDS. The result tile goes
-// through LDS, so bias, mask and C are read and written 16 bytes at a time.
+// One operand tile in registers, on its way to LDS. No load sits under a branch, so
+// the loads of the next K tile are all in flight during a tile's MFMAs. Rows past the
+// end of A or B repeat the last one (their results are not stored); K entries past
+// the end are zeroed on the way to LDS.
 //
 // In LDS the 16-byte chunk c of row n of a transposed operand sits at chunk
-// c ^ (n / 16 % 4): the operand is read row by row, 32 lanes along 256 contiguous bytes (with eight
-// rows per load, lanes across rows, every lane was a request of its own: dW of
-// 32,768 x 896 x 256 took 67 us), and its patches, 4 rows of the tile apart, then meet
-// on two lanes per bank instead of eight; the MFMA reads stay conflict-free.
-template <bool T>
-__device__ inline int gemm_chunk(const int row, const int c) {
-  return row * GLD + ((T ? c ^ (row >> 4 & 3) : c) << 3);
-}
-
-template <bool T>
-struct VecTile {
+// c ^ (n / 16 % 4): the operand is read row by row, 32 lanes along 256 contiguous
+// bytes (with eight rows per load, lanes across rows, every lane was a request of its
+// own: dW of 32,768 x 896 x 256 took 67 us), and its patches, 4 rows of the tile
+// apart, then meet on two lanes per bank instead of eight; the MFMA reads stay
+// conflict-free.
+template <bool T, int BK>
+struct Tile {
+  static constexpr int LD = BK + 8;                          // row stride in LDS
+  static constexpr int GCH = GBM * BK * 2 / 16 / GTHREADS;  // 16-byte chunks per thread
+  static __device__ inline int chunk(const int row, const int c) {
+    return row * LD + ((T ? c ^ (row >> 4 & 3) : c) << 3);
+  }
   u32x4 v[GCH];
+  // as whole vectors: 8 bytes of a transposed operand's rows, 16 of another's
   __device__ inline void load(const u16* __restrict__ X, const long ld, const int row0, const int nrows, const int k0,
                               const int kEnd) {
     const int t = threadIdx.x;
@@ -293,20 +132,54 @@ struct VecTile {
 #pragma unroll
       for (int i = 0; i < GCH; ++i) {
         const int c = t + GTHREADS * i;
-        const int gr = min(row0 + c / (GBK / 8), nrows - 1), gk = min(k0 + (c % (GBK / 8)) * 8, kEnd - 8);
+        const int gr = min(row0 + c / (BK / 8), nrows - 1), gk = min(k0 + (c % (BK / 8)) * 8, kEnd - 8);
         v[i] = *reinterpret_cast<const u32x4*>(X + (long)gr * ld + gk);
+      }
+    }
+  }
+  // Whether load() serves this tile of an operand whose rows start on whole vectors: the
+  // vectors of its contiguous dimension are whole inside it (the same for every thread).
+  static __device__ inline bool whole(const int row0, const int nrows, const int k0, const int kEnd) {
+    return T ? row0 + GBM <= nrows || nrows % 4 == 0 : k0 + BK <= kEnd || kEnd % 8 == 0;
+  }
+  // the same entries one by one; past an end the last one is read again, so that no load
+  // sits under a branch
+  __device__ inline void load_entries(const u16* __restrict__ X, const long ld, const int row0, const int nrows,
+                                      const int k0, const int kEnd) {
+    const int t = threadIdx.x;
+    if (T) {
+#pragma unroll
+      for (int ir = 0; ir < 2 * GCH; ++ir) {
+        const u16* x = X + (long)min(k0 + 32 * (ir >> 2) + 4 * (t >> 5) + (ir & 3), kEnd - 1) * ld;
+        unsigned e[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) e[j] = x[min(row0 + 4 * (t & 31) + j, nrows - 1)];
+        v[ir >> 1][2 * (ir & 1)] = e[0] | (e[1] << 16);
+        v[ir >> 1][2 * (ir & 1) + 1] = e[2] | (e[3] << 16);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < GCH; ++i) {
+        const int c = t + GTHREADS * i, gk = k0 + (c % (BK / 8)) * 8;
+        const u16* x = X + (long)min(row0 + c / (BK / 8), nrows - 1) * ld;
+        unsigned e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] = x[min(gk + j, kEnd - 1)];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] = gk + j < kEnd ? e[j] : 0u;
+        v[i] = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
       }
     }
   }
   __device__ inline void store(u16* __restrict__ s, const int k0, const int kEnd) {
     const int t = threadIdx.x;
-    if (k0 + GBK > kEnd) {  // the last K tile of a split: entries past the end are zero
+    if (k0 + BK > kEnd) {  // the last K tile of a split: entries past the end are zero
 #pragma unroll
       for (int i = 0; i < GCH; ++i)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           const int gk = T ? k0 + 32 * (i >> 1) + 4 * (t >> 5) + 2 * (i & 1) + h
-                           : k0 + ((t + GTHREADS * i) % (GBK / 8)) * 8;
+                           : k0 + ((t + GTHREADS * i) % (BK / 8)) * 8;
           if (gk >= kEnd) v[i][2 * h] = v[i][2 * h + 1] = 0u;
         }
     }
@@ -315,7 +188,7 @@ struct VecTile {
       for (int ij = 0; ij < 2 * GCH; ++ij) {
         const int i = ij >> 2, j = ij & 3, d = j >> 1;
         const unsigned pick = (j & 1) ? 0x07060302u : 0x05040100u;
-        u16* o = s + gemm_chunk<T>(4 * (t & 31) + j, 4 * i + (t >> 6)) + 4 * (t >> 5 & 1);
+        u16* o = s + chunk(4 * (t & 31) + j, 4 * i + (t >> 6)) + 4 * (t >> 5 & 1);
         *reinterpret_cast<u32x2*>(o) = u32x2{__builtin_amdgcn_perm(v[2 * i][2 + d], v[2 * i][d], pick),
                                              __builtin_amdgcn_perm(v[2 * i + 1][2 + d], v[2 * i + 1][d], pick)};
       }
@@ -323,7 +196,7 @@ struct VecTile {
 #pragma unroll
       for (int i = 0; i < GCH; ++i) {
         const int c = t + GTHREADS * i;
-        *reinterpret_cast<u32x4*>(s + gemm_chunk<T>(c / (GBK / 8), c % (GBK / 8))) = v[i];
+        *reinterpret_cast<u32x4*>(s + chunk(c / (BK / 8), c % (BK / 8))) = v[i];
       }
     }
   }
@@ -331,12 +204,19 @@ struct VecTile {
 
 constexpr int GCLD = GBN + 4;  // row stride of the result tile in LDS (FP32)
 
-template <bool TA, bool TB, int EPI>
-__global__ void __launch_bounds__(GTHREADS, 2) gemm_bf16_vec_kernel(const GemmArgs g) {
-  constexpr int ABYTES = 2 * 2 * GBM * GLD * 2, CBYTES = GBM * GCLD * 4;
+// VEC: every access of the product is a whole vector (gemm_vectors); the result tile
+// goes through LDS, so bias, mask and C are read and written 16 bytes at a time.
+// Otherwise each operand's tile takes vectors where its own rows allow them (an
+// unaligned result, or the other operand, does not change that) and the result is
+// written entry by entry: gathered to 128-byte runs through LDS first, 32,768 x 275 x
+// 125 took 69 us (data gradient) against 60.
+template <bool TA, bool TB, int EPI, bool VEC, int BK>
+__global__ void __launch_bounds__(GTHREADS, BK == 32 ? 3 : 2) gemm_bf16_kernel(const GemmArgs g) {
+  constexpr int LD = BK + 8;
+  constexpr int ABYTES = 2 * 2 * GBM * LD * 2, CBYTES = VEC ? GBM * GCLD * 4 : 0;
   __shared__ __attribute__((aligned(16))) char smem[ABYTES > CBYTES ? ABYTES : CBYTES];
   u16* const sA = reinterpret_cast<u16*>(smem);
-  u16* const sB = sA + 2 * GBM * GLD;
+  u16* const sB = sA + 2 * GBM * LD;
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
   const int wm = w >> 1, wn = w & 1;
   int mt, nt, split;
@@ -344,7 +224,7 @@ __global__ void __launch_bounds__(GTHREADS, 2) gemm_bf16_vec_kernel(const GemmAr
   const int m0 = mt * GBM, n0 = nt * GBN;
   const int kBeg = split * g.kChunk;
   const int kEnd = min(g.K, kBeg + g.kChunk);
-  const int nT = (kEnd > kBeg) ? (kEnd - kBeg + GBK - 1) / GBK : 0;
+  const int nT = (kEnd > kBeg) ? (kEnd - kBeg + BK - 1) / BK : 0;
 
   f32x16 acc[2][2];
 #pragma unroll
@@ -355,44 +235,81 @@ __global__ void __launch_bounds__(GTHREADS, 2) gemm_bf16_vec_kernel(const GemmAr
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
   const int lr = l & 31, lc = l >> 5;
   const auto product = [&](const int buf) {
-    const u16* a_s = sA + buf * GBM * GLD;
-    const u16* b_s = sB + buf * GBN * GLD;
+    const u16* a_s = sA + buf * GBM * LD;
+    const u16* b_s = sB + buf * GBN * LD;
 #pragma unroll
-    for (int ks = 0; ks < GBK; ks += 16) {
+    for (int ks = 0; ks < BK; ks += 16) {
       bf16x8 a[2], b[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        a[i] = *reinterpret_cast<const bf16x8*>(a_s + gemm_chunk<TA>(wm * 64 + i * 32 + lr, ks / 8 + lc));
+        a[i] = *reinterpret_cast<const bf16x8*>(a_s + Tile<TA, BK>::chunk(wm * 64 + i * 32 + lr, ks / 8 + lc));
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        b[j] = *reinterpret_cast<const bf16x8*>(b_s + gemm_chunk<TB>(wn * 64 + j * 32 + lr, ks / 8 + lc));
+        b[j] = *reinterpret_cast<const bf16x8*>(b_s + Tile<TB, BK>::chunk(wn * 64 + j * 32 + lr, ks / 8 + lc));
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
     }
   };
+  const bool vecA = VEC || (g.lda % 8 == 0 && ((uintptr_t)g.A & 15) == 0);
+  const bool vecB = VEC || (g.ldb % 8 == 0 && ((uintptr_t)g.B & 15) == 0);
+  const auto load = [&](auto& r, const u16* X, const long ld, const int row0, const int nrows, const int k0,
+                        const bool vec) {
+    if (VEC || (vec && r.whole(row0, nrows, k0, kEnd)))
+      r.load(X, ld, row0, nrows, k0, kEnd);
+    else
+      r.load_entries(X, ld, row0, nrows, k0, kEnd);
+  };
   if (nT > 0) {
-    VecTile<TA> ra;
-    VecTile<TB> rb;
-    ra.load(g.A, g.lda, m0, g.M, kBeg, kEnd);
-    rb.load(g.B, g.ldb, n0, g.N, kBeg, kEnd);
+    Tile<TA, BK> ra;
+    Tile<TB, BK> rb;
+    load(ra, g.A, g.lda, m0, g.M, kBeg, vecA);
+    load(rb, g.B, g.ldb, n0, g.N, kBeg, vecB);
     ra.store(sA, kBeg, kEnd);
     rb.store(sB, kBeg, kEnd);
     __syncthreads();
     for (int it = 0; it + 1 < nT; ++it) {
-      const int k0 = kBeg + (it + 1) * GBK;
-      ra.load(g.A, g.lda, m0, g.M, k0, kEnd);
-      rb.load(g.B, g.ldb, n0, g.N, k0, kEnd);
+      const int k0 = kBeg + (it + 1) * BK;
+      load(ra, g.A, g.lda, m0, g.M, k0, vecA);
+      load(rb, g.B, g.ldb, n0, g.N, k0, vecB);
       // all of the loads go out before the MFMAs: left to itself the scheduler spreads them
       // between, the last ones right before the stores that wait for them
       __builtin_amdgcn_sched_barrier(0);
       product(it & 1);
-      ra.store(sA + ((it & 1) ^ 1) * GBM * GLD, k0, kEnd);
-      rb.store(sB + ((it & 1) ^ 1) * GBN * GLD, k0, kEnd);
+      ra.store(sA + ((it & 1) ^ 1) * GBM * LD, k0, kEnd);
+      rb.store(sB + ((it & 1) ^ 1) * GBN * LD, k0, kEnd);
       __syncthreads();
     }
     product((nT - 1) & 1);
+  }
+  if constexpr (!VEC) {  // entry by entry
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int col = n0 + wn * 64 + j * 32 + lr;
+        if (col >= g.N) continue;
+        const float bcol = (g.bias && (EPI == EPI_F32_BIAS || EPI == EPI_BF16_BIAS_RELU)) ? g.bias[col] : 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int row = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
+          if (row >= g.M) continue;
+          const float v = acc[i][j][r];
+          if (EPI == EPI_F32_BIAS) {
+            const float o = v + bcol;
+            reinterpret_cast<float*>(g.C)[(long)row * g.ldc + col] = g.rowScale ? g.rowScale[row] * o : o;
+          } else if (EPI == EPI_BF16_BIAS_RELU) {
+            reinterpret_cast<u16*>(g.C)[(long)row * g.ldc + col] = f2bf(fmaxf(v + bcol, 0.f));
+          } else if (EPI == EPI_BF16_MASK) {
+            const bool keep = !g.mask || bf2f(g.mask[(long)row * g.ldm + col]) > 0.f;
+            reinterpret_cast<u16*>(g.C)[(long)row * g.ldc + col] = f2bf(keep ? v : 0.f);
+          } else {
+            reinterpret_cast<float*>(g.C)[(long)split * g.M * g.ldc + (long)row * g.ldc + col] = v;
+          }
+        }
+      }
+    return;
   }
   __syncthreads();  // the tiles have been read: the result tile takes their place
 
@@ -467,7 +384,7 @@ __global__ void __launch_bounds__(GTHREADS, 2) gemm_bf16_vec_kernel(const GemmAr
   }
 }
 
-// Whether gemm_bf16_vec_kernel serves the product: pointers and leading dimensions
+// Whether the VEC form serves the product: pointers and leading dimensions
 // whole vectors, the vectors of the contiguous dimension whole inside the matrix.
 template <bool TA, bool TB, int EPI>
 static bool gemm_vectors(const GemmArgs& g) {
@@ -484,10 +401,15 @@ template <bool TA, bool TB, int EPI>
 static int gemm(const GemmArgs& g, int splits, void* stream, const char* where) {
   if (g.M <= 0 || g.N <= 0) return LIBP_OK;
   dim3 grid((g.N + GBN - 1) / GBN, (g.M + GBM - 1) / GBM, splits);
-  if (gemm_vectors<TA, TB, EPI>(g))
-    hipLaunchKernelGGL((gemm_bf16_vec_kernel<TA, TB, EPI>), grid, dim3(GTHREADS), 0, as_stream(stream), g);
-  else
-    hipLaunchKernelGGL((gemm_bf16_kernel<TA, TB, EPI>), grid, dim3(GTHREADS), 0, as_stream(stream), g);
+  // Two workgroups of BK = 64 fit a CU, three of BK = 32: the smaller step where that takes one
+  // round over the 256 CUs instead of two (768 tiles: data gradient of 275 x 125 43 us against 60,
+  // forward 256 -> 343 25 against 33); elsewhere it is slower (512 tiles: forward 896 -> 256 with
+  // unaligned rows 136 us against 100).
+  const unsigned tiles = grid.x * grid.y * grid.z;
+  const auto kernel = gemm_vectors<TA, TB, EPI>(g)  ? gemm_bf16_kernel<TA, TB, EPI, true, GBK>
+                      : tiles > 512 && tiles <= 768 ? gemm_bf16_kernel<TA, TB, EPI, false, 32>
+                                                    : gemm_bf16_kernel<TA, TB, EPI, false, GBK>;
+  hipLaunchKernelGGL(kernel, grid, dim3(GTHREADS), 0, as_stream(stream), g);
   return launch_status(where);
 }
 

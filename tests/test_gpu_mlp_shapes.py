@@ -21,7 +21,9 @@ def product(a, b):
 
 
 @pytest.mark.parametrize("M,K,N", [(1, 8, 8), (5, 72, 24), (127, 64, 128), (128, 128, 128), (257, 136, 264),
-                                   (257, 150, 130), (300, 7, 9), (2055, 64, 256), (4099, 264, 136), (16411, 72, 8)])
+                                   (257, 150, 130), (300, 7, 9), (2055, 64, 256), (4099, 264, 136), (16411, 72, 8),
+                                   # 513 to 768 tiles of a forward layer, a data and a weight gradient
+                                   (21893, 50, 343), (21893, 343, 60), (10250, 1601, 99)])
 def test_mlp_products_at_tile_edges(M, K, N):
     L = lp.lib()
     g = torch.Generator(device="cuda")
@@ -67,3 +69,63 @@ def test_mlp_products_at_tile_edges(M, K, N):
     assert ((dW.double() - ref).abs() <= bound).all()
     mag = dY.double().abs().sum(0)
     assert ((db.double() - dY.double().sum(0)).abs() <= M * 2.0**-23 * mag).all()
+
+
+@pytest.mark.parametrize("pad,off", [(0, 0), (8, 0), (3, 0), (0, 1), (8, 4), (8, 8)])
+@pytest.mark.parametrize("M,K,N", [(5, 9, 4), (300, 136, 130), (300, 130, 136), (130, 260, 129), (513, 64, 343),
+                                   (300, 132, 256), (257, 250, 128)])
+def test_mlp_products_with_strides_and_offsets(M, K, N, pad, off):
+    """Rows longer than the width (a multiple of 8 and not) and operands `off` entries past an
+    aligned address: an operand is read in vectors or entry by entry tile by tile, together with
+    another that is not. What lies between the rows of an operand is NaN (it must not enter), and
+    between those of a result it stays."""
+    L = lp.lib()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + K + N + pad + off)
+    st = torch.cuda.current_stream().cuda_stream
+    nan = float("nan")
+
+    def rows(r, c, dtype=torch.bfloat16, fill=nan):
+        """An r x c view with row stride c + pad, `off` entries into its buffer."""
+        return torch.full((off + r * (c + pad),), fill, dtype=dtype, device="cuda")[off:].view(r, c + pad)[:, :c]
+
+    def operand(r, c):
+        v = rows(r, c)
+        v.copy_(torch.randn(r, c, device="cuda", generator=g))
+        return v
+
+    def close(got, want, bound):
+        torch.cuda.synchronize()
+        assert ((got.double() - want).abs() <= bound).all()
+        between = got.as_strided((got.shape[0], pad), got.stride(), got.storage_offset() + got.shape[1])
+        assert (between == 3.0).all()
+
+    X, W, dY, H = operand(M, K), operand(N, K), operand(M, N), operand(M, K)
+    lk, ln = K + pad, N + pad
+    b, scale = torch.randn(N, device="cuda", generator=g), torch.rand(M, device="cuda", generator=g) + 0.5
+    ref, bound = product(X, W.T)
+    bound = bound + 2.0**-22 * (ref.abs() + b.double().abs())
+    Y, Ys, Yr = rows(M, N, torch.float32, 3.0), rows(M, N, torch.float32, 3.0), rows(M, N, fill=3.0)
+    lp.check(L.libp_mlp_linear_fwd(M, K, N, X.data_ptr(), lk, W.data_ptr(), lk, b.data_ptr(), 0, Y.data_ptr(), ln, st))
+    close(Y, ref + b.double(), bound)
+    lp.check(L.libp_mlp_linear_fwd_scaled(M, K, N, X.data_ptr(), lk, W.data_ptr(), lk, None, scale.data_ptr(),
+                                          Ys.data_ptr(), ln, st))
+    close(Ys, scale.double()[:, None] * ref, 2 * bound)
+    lp.check(L.libp_mlp_linear_fwd(M, K, N, X.data_ptr(), lk, W.data_ptr(), lk, b.data_ptr(), 1, Yr.data_ptr(), ln, st))
+    relu = torch.relu(ref + b.double())
+    close(Yr, relu, bound + 2.0**-8 * relu)
+    ref, bound = product(dY, W)
+    for mask in (None, H):
+        dX = rows(M, K, fill=3.0)
+        lp.check(L.libp_mlp_linear_bwd_data(M, K, N, dY.data_ptr(), ln, W.data_ptr(), lk,
+                                            mask.data_ptr() if mask is not None else None, lk, dX.data_ptr(), lk, st))
+        want = ref if mask is None else torch.where(H.double() > 0, ref, 0.0)
+        close(dX, want, bound + 2.0**-8 * want.abs())
+    dW, db = torch.full((N, K), nan, device="cuda"), torch.full((N,), nan, device="cuda")
+    ws = torch.full((L.libp_mlp_ws_bytes(M, K, N) // 4,), nan, device="cuda")
+    lp.check(L.libp_mlp_linear_bwd_weight(M, K, N, dY.data_ptr(), ln, X.data_ptr(), lk, dW.data_ptr(), db.data_ptr(),
+                                          ws.data_ptr(), st))
+    torch.cuda.synchronize()
+    ref, bound = product(dY.T, X)
+    assert ((dW.double() - ref).abs() <= bound).all()
+    assert ((db.double() - dY.double().sum(0)).abs() <= M * 2.0**-23 * dY.double().abs().sum(0)).all()
