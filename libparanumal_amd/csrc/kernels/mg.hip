@@ -11,28 +11,54 @@
 //
 // The form before took a NqF x NqF tile per element (the same arithmetic and order,
 // bit for bit), read P from LDS for every product, left lanes idle (49 of 64 at
-// NqF = 7) and had known sizes at 7->3 and 3->1 only. What bounds this one: HBM (12
-// bytes per fine node with the weights, FP32), and for the restriction the latency
-// of its index -> value loads. 8M fine nodes, microseconds, restriction / prolongation
-// before and now:
-//             2->1      3->1      4->2      6->4      7->3      9->6     12->9     15->11
-//   FP64    105/106     61/32     42/41     52/38     39/15     50/53     54/63     56/83
-//      now   31/22      30/17     30/20     35/24     32/17     43/24     44/30     45/38
-//   FP32     92/101     45/30     32/38     35/31     26/9.8    34/36     31/35     32/42
-//      now   24/17      21/12     23/14     26/16     23/10.5   27/15     24/19     24/20
+// NqF = 7) and had known sizes at 7->3 and 3->1 only; it is left where it is the
+// faster one (mg_prolong_tile_kernel). What bounds this one: HBM (12 bytes per fine
+// node with the weights, FP32), and for the restriction the latency of its
+// index -> value loads. 8M fine nodes, microseconds, weighted restriction /
+// prolongation before and now (in turn on one card, ten launches in a replayed graph):
+//             2->1      3->1      4->2      6->4      7->3      9->8     12->9    15->11    15->14
+//   FP64   107/107     60/33     56/44     69/41     52/18     63/69     57/65     57/84    66/121
+//      now   28/23     31/19     32/21     39/26     38/16     53/36     44/32     42/39     58/53
+//   FP32    93/102     47/32     47/41     53/35     44/11     49/46     41/38     40/43     45/65
+//      now   27/18     25/14     28/15     31/18     31/12     42/24     34/21     32/23     35/29
+#include <type_traits>
+
 #include "kcommon.hpp"
 
 namespace libp_amd {
 
 // Elements and threads per workgroup: about 1000 nodes, and threads for all the
-// fine lines of one direction where that is a multiple of a wavefront or close to it.
-// 7->3 at 1 element / 64 threads, 2 / 128 and 4 / 256 prolongs in 17.6, 16.7 and
-// 16.7 us (FP64); the tile form took 15.3 there, and 40 against 33 to restrict.
+// fine lines of one direction where that is a multiple of a wavefront or close to it
+// (7->3 at 1 element / 64 threads, 2 / 128 and 4 / 256 prolongs in 17.6, 16.7 and 16.7 us).
 template <int NqF>
 struct MgShape {
   static constexpr int NE = NqF <= 3 ? 32 : NqF <= 5 ? 8 : NqF <= 7 ? 4 : NqF == 8 ? 2 : 1;
   static constexpr int threads = (NqF >= 8 && NqF <= 11) || NqF == 4 ? 128 : 256;
 };
+
+// out(c, sum_m P[m][c] x[m]), six c at a time: each row of P gives six neighbouring
+// entries per scalar load. One c at a time is NqF loads of a column, which the compiler
+// pipelines only where the count of c has a small factor (15->14 in FP64, 1728 elements:
+// 66 us as a tile, 80 so, 58 with six; 9->8 at 8 elements 6.0, 8.8 and 5.2; two, three
+// or four at a time are slower at Nq >= 9, eight alike).
+template <int NqF, int NqC, typename T, typename F>
+__device__ inline void mg_restrict_line(const T* __restrict__ P, const T (&x)[NqF], const F& out) {
+  constexpr int UC = 6;
+  const auto some = [&](const int c0, auto n) {
+    T res[n];
+#pragma unroll
+    for (int u = 0; u < n; ++u) res[u] = 0;
+#pragma unroll
+    for (int m = 0; m < NqF; ++m)
+#pragma unroll
+      for (int u = 0; u < n; ++u) res[u] += P[m * NqC + c0 + u] * x[m];
+#pragma unroll
+    for (int u = 0; u < n; ++u) out(c0 + u, res[u]);
+  };
+  if constexpr (NqC >= UC)
+    for (int c = 0; c + UC <= NqC; c += UC) some(c, std::integral_constant<int, UC>());
+  if constexpr (NqC % UC > 0) some(NqC - NqC % UC, std::integral_constant<int, NqC % UC>());
+}
 
 template <int NqF, int NqC, typename T>
 __global__ void __launch_bounds__(MgShape<NqF>::threads)
@@ -76,12 +102,7 @@ __global__ void __launch_bounds__(MgShape<NqF>::threads)
     T x[NqF];
 #pragma unroll
     for (int m = 0; m < NqF; ++m) x[m] = s_f[e * NpF + m * FF + ji];
-    for (int c = 0; c < NqC; ++c) {
-      T res = 0;
-#pragma unroll
-      for (int m = 0; m < NqF; ++m) res += P[m * NqC + c] * x[m];
-      s_c[(e * NqC + c) * FF + ji] = res;
-    }
+    mg_restrict_line<NqF, NqC>(P, x, [&](const int c, const T v) { s_c[(e * NqC + c) * FF + ji] = v; });
   }
   __syncthreads();
   // j: lines (e, k, i) of s_c -> s_f[e][k][c][i], rows of R
@@ -90,12 +111,7 @@ __global__ void __launch_bounds__(MgShape<NqF>::threads)
     T x[NqF];
 #pragma unroll
     for (int m = 0; m < NqF; ++m) x[m] = s_c[ek * FF + m * NqF + i];
-    for (int c = 0; c < NqC; ++c) {
-      T res = 0;
-#pragma unroll
-      for (int m = 0; m < NqF; ++m) res += P[m * NqC + c] * x[m];
-      s_f[(ek * NqC + c) * R + i] = res;
-    }
+    mg_restrict_line<NqF, NqC>(P, x, [&](const int c, const T v) { s_f[(ek * NqC + c) * R + i] = v; });
   }
   __syncthreads();
   // i: lines (e, k, j) of s_f -> s_c, flat coarse nodes
@@ -103,12 +119,7 @@ __global__ void __launch_bounds__(MgShape<NqF>::threads)
     T x[NqF];
 #pragma unroll
     for (int m = 0; m < NqF; ++m) x[m] = s_f[p * R + m];
-    for (int c = 0; c < NqC; ++c) {
-      T res = 0;
-#pragma unroll
-      for (int m = 0; m < NqF; ++m) res += P[m * NqC + c] * x[m];
-      s_c[p * NqC + c] = res;
-    }
+    mg_restrict_line<NqF, NqC>(P, x, [&](const int c, const T v) { s_c[p * NqC + c] = v; });
   }
   __syncthreads();
   const int NpC = NqC * NqC * NqC;
@@ -195,6 +206,54 @@ __global__ void __launch_bounds__(MgShape<NqF>::threads)
   }
 }
 
+// The prolongation with one wavefront per element, an 8 x 8 tile of its fine nodes, each
+// thread one (j, i). It keeps to itself (no barrier waits for another wave), which is
+// worth more than idle lanes while the coarse tile fills at most a quarter of it: 15,625
+// elements, FP64, 7->1, 7->2, 7->3 13.8, 14.8 and 16.5 us against 16.0, 17.6 and 18.4 in
+// mg_prolong_kernel, but 7->5 and 7->6 26.1 and 32.9 against 24.6 and 30.2 (7->4 alike).
+template <int NqC, typename T>
+__global__ void __launch_bounds__(64) mg_prolong_tile_kernel(const int* __restrict__ elementList,
+                                                             const int* __restrict__ G2LC, const T* __restrict__ P,
+                                                             const T* __restrict__ qcIn, T* __restrict__ qN) {
+  constexpr int NqF = 8;
+  __shared__ T s_A[NqC][NqF][NqF];  // coarse nodes, then the planes after the j sweep
+  __shared__ T s_ccf[NqC][NqC][NqF];
+  __shared__ T s_P[NqF][NqF - 1];
+  const size_t element = elementList ? elementList[blockIdx.x] : blockIdx.x;
+  const int t = threadIdx.x, i = t % NqF, j = t / NqF;
+  if (i < NqC && j < NqC) {
+    // index loads first, then unconditional value loads
+    int ids[NqC];
+#pragma unroll
+    for (int k = 0; k < NqC; ++k) ids[k] = G2LC[element * (NqC * NqC * NqC) + i + j * NqC + k * NqC * NqC];
+#pragma unroll
+    for (int k = 0; k < NqC; ++k) {
+      const T qv = qcIn[max(ids[k], 0)];
+      s_A[k][j][i] = (ids[k] >= 0) ? qv : T(0);
+    }
+  }
+  if (t < NqF * NqC) s_P[t / NqC][t % NqC] = P[t];
+  __syncthreads();
+  if (j < NqC)
+    for (int k = 0; k < NqC; ++k) {
+      T res = 0;
+      for (int m = 0; m < NqC; ++m) res += s_P[i][m] * s_A[k][j][m];
+      s_ccf[k][j][i] = res;
+    }
+  __syncthreads();
+  for (int k = 0; k < NqC; ++k) {
+    T res = 0;
+    for (int m = 0; m < NqC; ++m) res += s_P[j][m] * s_ccf[k][m][i];
+    s_A[k][j][i] = res;
+  }
+  __syncthreads();
+  for (int k = 0; k < NqF; ++k) {
+    T res = 0;
+    for (int m = 0; m < NqC; ++m) res += s_P[k][m] * s_A[m][j][i];
+    qN[element * (NqF * NqF * NqF) + i + j * NqF + k * NqF * NqF] = res;
+  }
+}
+
 // the kernel of coarse size nqc, NqC <= nqc < NqF
 template <int NqF, int NqC, typename T, bool COARSEN>
 static void launch_transfer(int nqc, int Nelements, const int* elist, const int* g2l, const T* P, const T* in,
@@ -204,6 +263,8 @@ static void launch_transfer(int nqc, int Nelements, const int* elist, const int*
     const dim3 grid((Nelements + MgShape<NqF>::NE - 1) / MgShape<NqF>::NE), block(MgShape<NqF>::threads);
     if constexpr (COARSEN)
       hipLaunchKernelGGL((mg_coarsen_kernel<NqF, NqC, T>), grid, block, 0, st, Nelements, elist, g2l, P, in, w, out);
+    else if constexpr (NqF == 8 && NqC <= 4)
+      hipLaunchKernelGGL((mg_prolong_tile_kernel<NqC, T>), dim3(Nelements), dim3(64), 0, st, elist, g2l, P, in, out);
     else
       hipLaunchKernelGGL((mg_prolong_kernel<NqF, NqC, T>), grid, block, 0, st, Nelements, elist, g2l, P, in, out);
   }

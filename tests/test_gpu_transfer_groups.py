@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("Nf,Nc", [(2, 1), (3, 1), (3, 2), (4, 2), (5, 4), (6, 4), (7, 3), (7, 5), (8, 1), (9, 6),
-                                   (11, 10), (12, 9), (13, 7), (15, 11), (15, 14)])
+                                   (11, 10), (12, 9), (13, 7), (15, 11), (15, 14),
+                                   # the 8 x 8 tile, and coarse lines of 5, 6, 7, 9, 12 and 13 in sixes
+                                   (7, 1), (7, 2), (7, 4), (6, 5), (10, 6), (9, 8), (12, 11), (14, 12)])
 def test_transfers_counts_and_lists(Nf, Nc):
     L = lp.lib()
     F, C = Nf + 1, Nc + 1
