@@ -18,19 +18,21 @@
 // factors of a thread's nodes are requested before the first barrier, so they
 // arrive while the contractions run. A thread tile per k-plane, with D in LDS
 // (the form this kernel replaces), made 8 Nq LDS reads per node and left
-// 64 - Nq^2 mod 64 lanes idle. Partial Ax of ~10M local nodes, lambda = 1,
-// curved boxes, microseconds before -> now (TB/s of those bytes now):
+// 64 - Nq^2 mod 64 lanes idle; here lanes idle only past the last pencil and the
+// last node of a group. Partial Ax of ~10M local nodes, lambda = 1, curved boxes,
+// microseconds before -> now (TB/s of those bytes now):
 //   N        1        2        3        4        5        6        7
-//   FP64  211->116 237->120 117->115 169->118 150->116 144->125   131
-//         (6.0)    (5.9)    (6.3)    (6.1)    (6.3)    (6.0)   (the tile)
-//   FP32  159->61  147->61   93->63  116->65   87->64   91->68   73->67
+//   FP64  211->116 237->119 117->115 169->118 150->121 144->124   131
+//         (6.0)    (5.9)    (6.3)    (6.1)    (6.1)    (6.0)   (the tile)
+//   FP32  159->61  147->62   93->63  116->65   87->64   91->69   73->67
 //   N        8        9       10       11       12       13       14
-//   FP64  144->121 181->127 146->137 204->123 166->162 204->124 203->145
-//         (6.1)    (6.2)    (5.8)    (6.1)    (4.9)    (5.5)    (4.8)
+//   FP64  144->121 181->127 146->137 204->123 166->147 204->124 203->145
+//         (6.1)    (6.2)    (5.8)    (6.1)    (5.5)    (5.5)    (4.8)
 //   FP32   93->67   90->72   84->73  106->69  116->80  107->72  101->80
 // (N = 15 FP32: 98->65; N = 7 in FP64 keeps the thread tile, see
-// ax_hex_tile_kernel; N = 15 in FP64 runs on the matrix cores, ax_hex_mfma.hip.) At N >= 12 in FP64 the LDS of an element (53-81 KB) leaves
-// two or three workgroups per CU, too few to cover the phases without loads.
+// ax_hex_tile_kernel; N = 15 in FP64 runs on the matrix cores, ax_hex_mfma.hip.)
+// At N >= 12 in FP64 the LDS of an element (53-81 KB) leaves two or three workgroups
+// per CU, too few to cover the phases without loads.
 //
 // Further:
 //  * elements run in natural order: brick or XCD-contiguous orderings that cut
@@ -61,7 +63,18 @@ namespace libp_amd {
 // per pass of a contraction's loop (UF: all of them while they fit the scalar
 // registers, two or three above), the nodes of a thread whose factors are
 // requested before the first barrier (GP), and whether the factors are read past the
-// caches. The shapes are the fastest of a sweep at ~10M nodes, lambda 0 and 1:
+// caches. The shapes are the fastest of a sweep at ~10M nodes, lambda 0 and 1, unless that
+// one was slower than the tile at another size between 20 thousand and 55M nodes:
+//  * Nq = 8 in FP32: two elements with all of D in scalar registers (33^3 elements,
+//    lambda 0 / 1: 112 / 122 us, 48^3 324 / 360) and not one element with two rows of D
+//    at a time (124 / 134 and 365 / 397; the tile 117 / 124 and 322 / 346);
+//  * Nq = 3, 6 and 7: more threads per element, or all of D (FP32, 14^3 elements of
+//    Nq = 3 4.6 -> 3.9 us, the tile 4.0; 4^3 of Nq = 7 7.3 -> 6.3, the tile 6.9).
+// What is left: 10^3 elements of Nq = 11 (FP64, lambda = 1) 23.2 us, the tile 21.9: their
+// workgroups take two rounds where the tile's took one, and the shapes with four
+// workgroups per CU lose 2 to 6% from 4M nodes on (the PAP form of Nq = 13 there: 49.8
+// and 46.4); Nq = 8 in FP32 at 48^3, lambda = 1, as above; 0.3 us at Nq = 2 below 5000 elements.
+// The rules of the sweep:
 //  * T is a multiple of 256 where an element has over 64 pencils: five to seven waves
 //    per workgroup spread unevenly over the four SIMDs (Nq = 12, 320 threads: 264 us
 //    against 123 with 256);
@@ -85,7 +98,7 @@ template <> struct AxShape<3, double> : AxShapeOf<8, 128, 2, 3, ALL, false> {};
 template <> struct AxShape<4, double> : AxShapeOf<4, 64, 2, 4, ALL, true> {};
 template <> struct AxShape<5, double> : AxShapeOf<4, 256, 2, 5, ALL, true> {};
 template <> struct AxShape<6, double> : AxShapeOf<4, 256, 2, 6, ALL, true> {};
-template <> struct AxShape<7, double> : AxShapeOf<2, 256, 2, 2, ALL, true> {};
+template <> struct AxShape<7, double> : AxShapeOf<2, 256, 2, 7, ALL, true> {};
 template <> struct AxShape<9, double> : AxShapeOf<1, 256, 2, 3, ALL, true> {};
 template <> struct AxShape<10, double> : AxShapeOf<1, 256, 2, 5, ALL, true> {};
 template <> struct AxShape<11, double> : AxShapeOf<1, 256, 2, 2, ALL, true> {};
@@ -95,12 +108,12 @@ template <> struct AxShape<14, double> : AxShapeOf<1, 512, 4, 2, 4, true> {};
 template <> struct AxShape<15, double> : AxShapeOf<1, 512, 4, 1, 4, true> {};
 template <> struct AxShape<16, double> : AxShapeOf<1, 512, 2, 2, ALL, true> {};  // the E-vector form only
 template <> struct AxShape<2, float> : AxShapeOf<64, 128, 2, 2, ALL, false> {};
-template <> struct AxShape<3, float> : AxShapeOf<8, 64, 2, 3, ALL, false> {};
+template <> struct AxShape<3, float> : AxShapeOf<16, 256, 2, 3, ALL, false> {};
 template <> struct AxShape<4, float> : AxShapeOf<8, 128, 2, 4, ALL, true> {};
 template <> struct AxShape<5, float> : AxShapeOf<4, 256, 2, 5, ALL, false> {};
-template <> struct AxShape<6, float> : AxShapeOf<4, 256, 2, 2, ALL, false> {};
-template <> struct AxShape<7, float> : AxShapeOf<4, 256, 2, 2, ALL, false> {};
-template <> struct AxShape<8, float> : AxShapeOf<1, 128, 2, 2, ALL, true> {};
+template <> struct AxShape<6, float> : AxShapeOf<4, 256, 2, 6, ALL, false> {};
+template <> struct AxShape<7, float> : AxShapeOf<4, 256, 2, 7, ALL, false> {};
+template <> struct AxShape<8, float> : AxShapeOf<2, 256, 2, 8, ALL, true> {};
 template <> struct AxShape<9, float> : AxShapeOf<1, 256, 2, 3, ALL, false> {};
 template <> struct AxShape<10, float> : AxShapeOf<1, 256, 2, 2, ALL, false> {};
 template <> struct AxShape<11, float> : AxShapeOf<1, 256, 2, 2, ALL, false> {};
@@ -109,6 +122,18 @@ template <> struct AxShape<13, float> : AxShapeOf<1, 512, 2, 2, ALL, false> {};
 template <> struct AxShape<14, float> : AxShapeOf<1, 256, 2, 2, ALL, false> {};
 template <> struct AxShape<15, float> : AxShapeOf<1, 512, 4, 2, ALL, false> {};
 template <> struct AxShape<16, float> : AxShapeOf<1, 512, 4, 4, ALL, false> {};
+
+// The waves and GP of an instance, elsewhere those of the shape (NE and threads stay: the
+// launcher counts blocks by them). At Nq = 13 the mass term takes the E-vector form past 168
+// registers, two workgroups per CU; with seven of nine nodes early three fit (9^3 elements,
+// lambda = 1, 34.5 -> 27.8 us, the tile 31.7; 15^3 118 -> 106). The list form keeps ALL (29^3
+// 716 against 803 us), and the split form (862 against 950). At Nq = 11 the split form is faster with
+// four workgroups per CU (10^3 elements, lambda 0 / 1, 27.9 / 28.9 -> 25.3 / 26.6 us, the
+// tile 25.4 / 25.1; 18^3 112 / 122 -> 106 / 116), the E-vector form is not (95 -> 98).
+template <int Nq, typename R, int OUT, bool LAM, bool LIST>
+struct AxInstance : AxShape<Nq, R> {};
+template <> struct AxInstance<13, double, 0, true, false> : AxShapeOf<1, 256, 3, 1, 7, true> {};
+template <bool LAM> struct AxInstance<11, double, 1, LAM, false> : AxShapeOf<1, 256, 4, 2, 4, true> {};
 
 // Number of element-boundary nodes of an Nq^3 element, and the position of
 // node (i,j,k) among them in local order (the node index minus the interior
@@ -203,7 +228,7 @@ __device__ inline void ax_contract(const R* __restrict__ D, const R* src, R* dst
 // values stored by several threads of the one block.
 template <int Nq, typename R, int MODE, int OUT, bool PAP, bool LAM, bool LIST>
 __global__ void __launch_bounds__((AxShape<Nq, R>::threads))
-    __attribute__((amdgpu_waves_per_eu((AxShape<Nq, R>::waves))))
+    __attribute__((amdgpu_waves_per_eu((AxInstance<Nq, R, OUT, LAM, LIST>::waves))))
     ax_hex_kernel(const int Nelements, const int* __restrict__ elementList, const int* __restrict__ G2L,
                   const R* __restrict__ wJ, const R* __restrict__ ggeo, const R* __restrict__ D, const R lambda,
                   const R* __restrict__ q, R* __restrict__ Aq, R* __restrict__ Ag, double* __restrict__ pap,
@@ -213,7 +238,7 @@ __global__ void __launch_bounds__((AxShape<Nq, R>::threads))
   // contraction across expressions the backend may fuse x*y + z*w as
   // fma(x, y, z*w) in one instantiation and fma(z, w, x*y) in another
 #pragma clang fp contract(on)
-  using S = AxShape<Nq, R>;
+  using S = AxInstance<Nq, R, OUT, LAM, LIST>;
   using L = AxLds<Nq>;
   using offset = std::conditional_t<LIST, size_t, unsigned>;
   constexpr int NE = S::NE, T = S::threads, UF = S::UF, GP = S::GP;

@@ -18,7 +18,7 @@ from tests.oracle_lib import OracleElliptic
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("N", [1, 2, 3, 4, 6, 7, 8, 10, 13, 14, 15])
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 13, 14, 15])
 def test_ax_counts_and_lists(N):
     shape = (5, 4, 4) if N <= 4 else (3, 2, 1)
     o = OracleElliptic({"MESH FILE": "BOX", "MESH DIMENSION": 3, "ELEMENT TYPE": 12, "BOX NX": shape[0],
