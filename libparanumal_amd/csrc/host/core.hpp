@@ -223,7 +223,7 @@ class platform_t {
   // Device memory for work on this platform's stream, kept for the next caller of the same
   // size when its last holder lets go of it: a solve's vectors (elliptic_t::Run makes about
   // a dozen) cost ~0.15 ms each to allocate and free, 1.9 of the 10.2 ms of a whole p-MG
-  // call on 2.9M nodes. Reuse is ordered by the stream. At most 16 buffers and 512 MiB
+  // call on 2.9M nodes. Reuse is ordered by the stream. At most 16 buffers and 1 GiB
   // wait (the oldest are freed); all are freed with the platform, or when an allocation
   // finds no memory.
   template <typename T>

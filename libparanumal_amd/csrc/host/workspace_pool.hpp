@@ -14,10 +14,10 @@ namespace libp {
 
 class workspacePool {
  public:
-  // A p-MG solve on 2.9M nodes lets go of about 200 MB in a dozen buffers. From the
-  // sizes at which its vectors no longer fit here, allocating them is a small share of a
-  // solve (40^3 elements, N = 7: 2.0 GB would wait; 6.1 ms of a run become 8.0).
-  static constexpr size_t MOST = 16, MOST_BYTES = size_t(512) << 20;
+  // The vectors of a 32^3, N = 7 solve (16.8M nodes) fit: with half of this its p-MG run took
+  // 21.1 ms and not 19.7. From there on allocating is a small share of a solve (40^3: 2.0 GB
+  // would wait, and 6.1 ms beside the iterations become 7.7).
+  static constexpr size_t MOST = 16, MOST_BYTES = size_t(1) << 30;
   using release_t = void (*)(void*);
 
   explicit workspacePool(release_t release_) : release(release_) {

@@ -44,11 +44,11 @@ def test_handle_keeps_little_after_a_solve_and_repeats_it():
     el.run()
     kept = before - free()
     evector = 8 * 40**3 * 512
-    assert kept <= evector + (512 << 20) + (64 << 20), kept
+    assert kept <= evector + (1 << 30) + (64 << 20), kept
     x = el.solution()
     el.run()
     assert np.array_equal(el.solution(), x)
-    assert before - free() <= evector + (512 << 20) + (64 << 20)
+    assert before - free() <= evector + (1 << 30) + (64 << 20)
     el.close()
     for solver in ("PCG", "NBPCG", "NBFPCG", "FPCG"):
         small = handle(5, 4, **{"LINEAR SOLVER": solver})

@@ -49,7 +49,6 @@ static void expect(bool ok, const char* what) {
 }
 
 int main() {
-  const size_t MB = size_t(1) << 20;
   {  // the last buffer given of a size comes back, no other size
     workspacePool pool(deviceFree);
     void *a = workspace(pool, 8), *b = workspace(pool, 8);
@@ -76,14 +75,15 @@ int main() {
   expect(used == 0, "freed with the pool (2)");
   {  // at most MOST_BYTES wait; a buffer above them is freed and leaves the others
     workspacePool pool(deviceFree);
+    const size_t part = workspacePool::MOST_BYTES / 5 * 2;  // two fit
     void* p[4];
-    for (void*& q : p) q = workspace(pool, 200 * MB);
+    for (void*& q : p) q = workspace(pool, part);
     void* big = workspace(pool, workspacePool::MOST_BYTES + 1);
-    for (void* q : p) pool.give(q, 200 * MB);
-    expect(used - (workspacePool::MOST_BYTES + 1) == 400 * MB, "bytes");
+    for (void* q : p) pool.give(q, part);
+    expect(used - (workspacePool::MOST_BYTES + 1) == 2 * part, "bytes");
     pool.give(big, workspacePool::MOST_BYTES + 1);
-    expect(used == 400 * MB && pool.take(200 * MB) == p[3], "above the limit");
-    pool.give(p[3], 200 * MB);
+    expect(used == 2 * part && pool.take(part) == p[3], "above the limit");
+    pool.give(p[3], part);
     void* whole = workspace(pool, workspacePool::MOST_BYTES);
     pool.give(whole, workspacePool::MOST_BYTES);
     expect(used == workspacePool::MOST_BYTES, "a buffer of the limit displaces the others");
