@@ -5,7 +5,7 @@
 //  * flat: thread t holds the nodes t, t + T, ... of the group in local order.
 //    The index map, the values, the geometric factors and the result are read
 //    and written this way, so every access to HBM is a run of consecutive
-//    entries whatever the degree, and no lane is idle;
+//    entries whatever the degree, and lanes idle only past the end of a group;
 //  * pencils: a thread holds one whole line of Nq nodes along r, s or t and
 //    contracts it with D. D[o][m] is then the same for every lane, so it comes
 //    through scalar loads and each node costs one LDS read and one LDS write
@@ -64,16 +64,19 @@ namespace libp_amd {
 // registers, two or three above), the nodes of a thread whose factors are
 // requested before the first barrier (GP), and whether the factors are read past the
 // caches. The shapes are the fastest of a sweep at ~10M nodes, lambda 0 and 1, unless that
-// one was slower than the tile at another size between 20 thousand and 55M nodes:
-//  * Nq = 8 in FP32: two elements with all of D in scalar registers (33^3 elements,
-//    lambda 0 / 1: 112 / 122 us, 48^3 324 / 360) and not one element with two rows of D
-//    at a time (124 / 134 and 365 / 397; the tile 117 / 124 and 322 / 346);
-//  * Nq = 3, 6 and 7: more threads per element, or all of D (FP32, 14^3 elements of
-//    Nq = 3 4.6 -> 3.9 us, the tile 4.0; 4^3 of Nq = 7 7.3 -> 6.3, the tile 6.9).
-// What is left: 10^3 elements of Nq = 11 (FP64, lambda = 1) 23.2 us, the tile 21.9: their
-// workgroups take two rounds where the tile's took one, and the shapes with four
-// workgroups per CU lose 2 to 6% from 4M nodes on (the PAP form of Nq = 13 there: 49.8
-// and 46.4); Nq = 8 in FP32 at 48^3, lambda = 1, as above; 0.3 us at Nq = 2 below 5000 elements.
+// one was slower than the tile at another size between 20 thousand and 55M nodes: more
+// threads per element, or all of D, at Nq = 3, 6 and 7 (FP32, 14^3 elements of Nq = 3
+// 4.6 -> 3.9 us, the tile 4.0; 4^3 of Nq = 7 7.3 -> 6.3, the tile 6.9).
+// What is left, each against the tile:
+//  * Nq = 8 in FP32, the kernel called over and over with nothing between: from 16M nodes 6 to
+//    14% slower (33^3, lambda = 0, 124 us against 117). Two elements per workgroup mend
+//    that (110 us) and lose where the kernel is used, between the gathers of a smoother:
+//    32^3, three handles in turn, 587 us per smoothing against 580, 40^3 1191 against 1146
+//    (the tile 581 and 1167; in the trace of one handle the Ax 104 us in both, the tile 120);
+//  * 10^3 elements of Nq = 11 (FP64, lambda = 1) 23.2 us and 21.9: their workgroups take two
+//    rounds where the tile's took one, and shapes with four workgroups per CU lose 2 to 6%
+//    from 4M nodes on (likewise the PAP form of Nq = 13, 49.8 and 46.4);
+//  * 0.3 us at Nq = 2 below 5000 elements.
 // The rules of the sweep:
 //  * T is a multiple of 256 where an element has over 64 pencils: five to seven waves
 //    per workgroup spread unevenly over the four SIMDs (Nq = 12, 320 threads: 264 us
@@ -113,7 +116,7 @@ template <> struct AxShape<4, float> : AxShapeOf<8, 128, 2, 4, ALL, true> {};
 template <> struct AxShape<5, float> : AxShapeOf<4, 256, 2, 5, ALL, false> {};
 template <> struct AxShape<6, float> : AxShapeOf<4, 256, 2, 6, ALL, false> {};
 template <> struct AxShape<7, float> : AxShapeOf<4, 256, 2, 7, ALL, false> {};
-template <> struct AxShape<8, float> : AxShapeOf<2, 256, 2, 8, ALL, true> {};
+template <> struct AxShape<8, float> : AxShapeOf<1, 128, 2, 2, ALL, true> {};
 template <> struct AxShape<9, float> : AxShapeOf<1, 256, 2, 3, ALL, false> {};
 template <> struct AxShape<10, float> : AxShapeOf<1, 256, 2, 2, ALL, false> {};
 template <> struct AxShape<11, float> : AxShapeOf<1, 256, 2, 2, ALL, false> {};
