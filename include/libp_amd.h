@@ -278,8 +278,9 @@ int libp_pcg_gather_jacobi_update_f64(int Nrows, const int* rowStarts, const int
  * libp_pcg_ax_hex_pap_f64 and libp_pcg_gather_jacobi_update_f64, bit for bit.
  * states holds two blocks of 16 doubles in the layout of the scalars, zeroed before
  * the first iteration (it = 0) except states[16 + RDOTZ1] = r.z (libp_pcg_jacobi_rdotz_f64
- * with scalars = states + 16) and states[16 + TOL]; iteration it leaves its scalars in
- * block it & 1 and does nothing once STOP is set. papPartials and gatherPartials are
+ * with scalars = states + 16) and states[16 + TOL]; iteration it leaves r.z, its
+ * predecessor, beta, r.r, TOL, STOP and the count in block it & 1 (ALPHA and PAP stay zero:
+ * the kernels form them for themselves) and does nothing once STOP is set. papPartials and gatherPartials are
  * sized as for the two calls. _check writes the scalars after iteration it (RDOTZ1, RDOTR,
  * TOL, STOP, ITERS) into pinned host memory mapped for the device. */
 int libp_pcg_jacobi_iteration_folds(int N, int Nelements, int Nrows);

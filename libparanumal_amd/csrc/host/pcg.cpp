@@ -81,8 +81,9 @@ void pcg::iteration(operator_t& linearOperator, operator_t& precon, diagonalPrec
  * (operator_t::JacobiPCGIteration), the same iterates and stopping test. A check
  * kernel behind each chunk writes the scalars to mapped host memory, and the next
  * chunk is queued before the host waits for it; iterations queued past the tolerance
- * do nothing. (8^3 elements, N = 4, 160 iterations, five launches per iteration and a
- * wait after every fourth took 4.13 ms for the whole run, 2.85 ms in this form.) */
+ * do nothing. (8^3 elements, N = 4, 160 iterations: five launches per iteration and a
+ * wait after every fourth took 4.76 ms for the whole run, 2.98 ms in this form; three
+ * handles in turn.) */
 int pcg::solveFolded(operator_t& A, diagonalPrecon_t& jac, deviceMemory<dfloat>& o_x, deviceMemory<dfloat>& o_r,
                      dfloat TOL, int MAXIT) {
   void* st = platform.s();
