@@ -541,7 +541,7 @@ constexpr int CSR_LANES = 8, CSR_UNROLL = 32 / CSR_LANES;
 // 29,791 rows, 233 blocks of 1024 threads beat 466 of 512 and 932 of 256), but below 256
 // blocks CUs are left idle while the others issue more of the divergent column loads:
 // the smallest block that gives at most 256 of them. 4,845 rows: 38 blocks of 1024 threads
-// took 9.1 us per iteration, 152 of 256 take 6.2 us (kernel trace; the three block sums behind one barrier).
+// took 9.1 us per iteration, 152 of 256 take 6.2 to 6.5 us (kernel traces; the three block sums behind one barrier).
 static int csr_threads(int Nrows) {
   return Nrows <= 256 * (256 / CSR_LANES) ? 256 : Nrows <= 256 * (512 / CSR_LANES) ? 512 : 1024;
 }
